@@ -336,7 +336,7 @@ long long dnsmi_pnet_params(int din, int H, int dout); /* -1 if unsupported */
 /* Gradient of L = (1/(B dout)) sum (Y - T)^2 over X (B,din) bf16, T (B,dout)
  * FP32 into grad (FP32), loss into loss_dev (may be NULL).  Work: wf
  * B (2H + dout) floats, wh B (3H + dout) words, part ceil(B dout/256)
- * floats. */
+ * floats (not used: the partial sums live in wf). */
 int dnsmi_pnet_grad(int din, int H, int dout, int B, const void* X, const float* T, const float* params,
                     void* wb, float* wf, void* wh, float* part, float* grad, float* loss_dev, void* stream);
 /* Y (B,dout) = net(X); work wf 2 H B floats, wh 2 H B words. */
