@@ -236,7 +236,8 @@ int dnsmi_mlp_sizes(int H, long long* nparams, long long* packed_weight_bytes,
                     long long* bias_floats);
 /* Gradient of L = (1/B) sum (y - t)^2 over X (B,16), T (B,6), FP32, samples
  * summed in a fixed order (deterministic).  part: (ceil(B/32) +
- * ceil(B/1024)) * (nparams + 1) floats of scratch; grad: nparams floats;
+ * ceil(B/1024)) * (nparams + 1) floats of scratch (a caller's workspace for
+ * any B; at most 1024 rows of it are used); grad: nparams floats;
  * loss_dev: 1 float or NULL.
  * bf16 != 0 rounds weights and layer inputs to bfloat16 as inference does
  * (straight-through gradients). */
@@ -245,7 +246,7 @@ int dnsmi_mlp_grad(int H, int B, const float* X, const float* T, const float* pa
 /* dnsmi_mlp_grad without the `part` workspace and without any device
  * allocation.  No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under graph capture, serving loops).
- * The scratch is a file-scope device array of 6.0 MB per GPU (held until
+ * The scratch is a file-scope device array of 5.8 MB per GPU (held until
  * the process ends), which limits a call to B <= 8192 samples (larger B:
  * DNSMI_EINVAL).  Every call on one GPU shares that array: calls that overlap
  * on one GPU (other streams, other threads) race.  Same kernels and sums as
