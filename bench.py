@@ -817,7 +817,7 @@ def walls_large_form(steps: int, collect_steps: int = 8, train_iters: int = 300,
 def profile_imm(calls: int) -> None:
     """The plane Couette influence-matrix step (predict: one IMM on the
     state's RHS) in the three band-solve forms (chunk maps in five launches
-    or fused into two, sequential sweeps),
+    or fused into one, sequential sweeps),
     at 64x128x64 (p=4) and 128x256x128 (p=6), `calls` timed calls each after
     five warm-up calls; prints the time per call, a checksum of the result
     (equal for both forms up to rounding) and the autotuner's choice."""

@@ -13,11 +13,12 @@
 //   RHS (flows/plane_couette.py:274-289): WT1 FD curl + transpose
 //   (3,Nkz,Nkx,Ny) -> 6 fields (Ny,Nkz,Nkx); z-inverse; the shared x pass
 //   with base flow U = y; the shared z-forward; WT5 transpose back.
-//   IMM (flows/plane_couette.py:376-504): one thread per (kz, kx) mode
-//   streams over y: divergence and Lk d, the Lk forward sweep fed on the
-//   fly, back substitution, the three Hk right-hand sides fed into one
-//   forward sweep, back substitution, wall divergence, alpha = -M^-1 d,
-//   assembly, correction and the quadrature-weighted norm partials.
+//   IMM (flows/plane_couette.py:376-504): divergence, the pressure's Lk
+//   solve, the three velocity solves with Hk, wall divergence, alpha = -M^-1 d,
+//   correction and the quadrature-weighted norm partials: one launch whose
+//   workgroups take two modes of one k^2 class each, band solves as chains of
+//   matrix-core products (k_imm_fused); the same in five launches, or with
+//   sequential sweeps, where the modes are too few or the columns too long.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -47,6 +48,7 @@ struct WallTables {
   int curl_ty = 32;  // y points per curl workgroup (walls_curl_ty)
   // device
   double* d1w = nullptr;  // (Ny, p+1)
+  double *d1t = nullptr, *d2t = nullptr;  // the same as (p+1, Ny), (p+2, Ny): lanes along y read adjacent words
   int* d1j0 = nullptr;    // (Ny)
   double* d2w = nullptr;  // (Ny, p+2)
   int* d2j0 = nullptr;
@@ -62,10 +64,11 @@ struct WallTables {
   double* mkz = nullptr;
   double* scratch = nullptr;  // IMM work vectors, complex [vec][mode][y]
   // chunk maps of the band solves (chunked sweeps), one per distinct k^2,
-  // packed (map_offset); sched = the modes, with their maps, in the order
-  // the chunked solve takes them (two per wavefront)
+  // (map_word); sched = the modes, with their maps, in the order
+  // the chunked solve takes them (items of two modes of one map)
   double *lk_fmap = nullptr, *lk_bmap = nullptr, *hk_fmap = nullptr, *hk_bmap = nullptr;
-  int2* sched = nullptr;  // (mode, map) per slot
+  int2* sched = nullptr;  // (mode, map) per slot, two slots per item
+  int items = 0;
   int U = 0;              // distinct k^2 values
   // host copies: the y grid, and each mode's class (walls_table reads the
   // device tables back in the reference layouts through it)
@@ -207,94 +210,91 @@ static void band_solve(const Band& B, std::vector<double>& b) {
   }
 }
 
-// Rows per chunk of the chunked band solve, and the register slots of its
-// map prefetch (a chunk's map is loaded kChunkSlots - 1 chunks ahead).
-constexpr int kChunk = 16;
-constexpr int kChunkSlots = 3;
-// two slots where three would spill (fd_order 8, three right-hand sides)
-constexpr int chunk_slots(int po, int nr) { return po == 8 && nr == 3 ? 2 : kChunkSlots; }
-// window words read from LDS per batch: two where eight would not leave
-// two waves per SIMD without spilling (one right-hand side, fd_order >= 6)
-constexpr int window_batch(int po, int nr) { return nr == 1 && po >= 6 ? 2 : 8; }
-// waves per SIMD the chunked solve asks for: two with one right-hand side
-// (registers within 256) up to fd_order 6, else one
-constexpr int chunk_waves(int po, int nr) { return nr == 1 && po <= 6 ? 2 : 1; }
-
-// Packed chunk maps.  Entry (t, k) of a map (out_t = sum_k map[t][k] w_k)
-// is zero by construction for k > t + lag: lag = kl for a forward map (a
-// row swap or elimination at window row t reaches at most kl rows down),
-// lag = 0 for a back map (row t draws only on the rows solved before it).
-// Column k of a map is therefore stored as one zero word (read by the rows
-// t < map_lo(k)) followed by rows map_lo(k) .. w-1, map_len(k) words in
-// all; the maps' columns lie side by side: chunk c, column k, map u, row t
-// at map_offset (lanes t of one map read consecutive words).
-__host__ __device__ constexpr int map_lo(int k, int lag) { return k > lag ? k - lag : 0; }
-__host__ __device__ constexpr int map_len(int k, int lag, int w) { return w - map_lo(k, lag) + 1; }
-// words of columns 0 .. k-1
-__host__ __device__ constexpr int map_pre(int k, int lag, int w) {
-  return k * (w + 1) - (k > lag + 1 ? (k - lag - 1) * (k - lag) / 2 : 0);
+// Chunk maps of the band solves: a chunk of B rows, with the rows its steps
+// reach (kl after it forward, kl + ku before it back), is a window of at most
+// 16 rows, or of 32 where a back window's reach leaves 16 too little (p >= 6).
+// B is a multiple of four rows, so that the rows a window keeps move by whole
+// registers of the matrix cores' operands (chunk_chain).
+__host__ __device__ constexpr int chunk_tiles(int p, bool back) { return back && p >= 6 ? 2 : 1; }
+__host__ __device__ constexpr int chunk_rows(int p, bool back) {
+  return 16 * chunk_tiles(p, back) - ((back ? 2 * p : p) + 3) / 4 * 4;
 }
-// word of row t (t < w) of column k of map u within one chunk's maps
-__host__ __device__ constexpr int map_word_at(int k, int u, int t, int lag, int w, int U) {
-  return U * map_pre(k, lag, w) + u * map_len(k, lag, w) + (t >= map_lo(k, lag) ? 1 + t - map_lo(k, lag) : 0);
+__host__ __device__ constexpr int chunk_window(int p, bool back) { return chunk_rows(p, back) + (back ? 2 * p : p); }
+__host__ __device__ constexpr int chunk_count(int n, int p, bool back) {
+  return (n + chunk_rows(p, back) - 1) / chunk_rows(p, back);
 }
-__host__ __device__ inline size_t map_offset(int c, int k, int u, int t, int lag, int w, int U) {
-  return (size_t)c * U * map_pre(w, lag, w) + (size_t)map_word_at(k, u, t, lag, w, U);
+// A map's words, in the order the products take them (map of chunk c, class
+// u at (c U + u) words): operand e of lane (g = lane / 16, r = lane % 16) at
+// map_word(e, lane), two operands side by side, so that a wavefront's load
+// is 1 KB of consecutive words.  One tile: e = k / 4, entry (t = r, k = 4 e +
+// g).  Two: e < 8 rows 16 + r, e = 8 .. 11 rows r, of which k >= 16 is zero by
+// construction (a back map is lower triangular) and left out.
+__host__ __device__ constexpr int map_operands(int p, bool back) { return chunk_tiles(p, back) == 1 ? 4 : 12; }
+__host__ __device__ constexpr int map_words(int p, bool back) { return 64 * map_operands(p, back); }
+__host__ __device__ constexpr int map_word(int e, int lane) { return ((e >> 1) * 64 + lane) * 2 + (e & 1); }
+// entry (t, k) of word i, and back: -1 where it is left out
+__host__ __device__ inline void map_entry(int i, bool two, int& t, int& k) {
+  const int e = (i >> 7) * 2 + (i & 1), lane = (i & 127) >> 1;
+  t = (lane & 15) + (two && e < 8 ? 16 : 0);
+  k = 4 * (two && e >= 8 ? e - 8 : e) + (lane >> 4);
 }
 
 // Chunk maps of one band solve (the operation order of band_solve): forward
 // chunk c applies the steps j in [cB, min(cB + B, n - 1)) (row swap,
-// elimination) to the window of rows cB + t, t < WF = B + kl; its map F_c is
-// those row operations applied to the identity.  Back chunk c, top row
-// T = n - 1 - cB, applies the steps j = T, T - 1, ... (at most B, j >= 0:
-// divide by the diagonal, eliminate upwards) to the window of rows T - t,
-// t < WB = B + kl + ku.  Written packed as map u of U; `raw(r, j)` reads
-// the factored band, `piv(j)` the pivot row.  Returns false if an entry
-// outside the packed region is not zero (it cannot be, by the argument
-// above; the check keeps the packing honest).
+// elimination) to the window of rows cB + t, t < W = B + kl; its map is those
+// row operations applied to the identity.  Back chunk c, top row T = n - 1 -
+// cB, applies the steps j = T, T - 1, ... (at most B, j >= 0: divide by the
+// diagonal, eliminate upwards) to the window of rows T - t, t < W = B + kl +
+// ku.  Written as map u of U; `raw(r, j)` reads the factored band, `piv(j)`
+// the pivot row.  Returns false if an entry left out is not zero (it cannot
+// be, by the argument above; the check keeps the layout honest).
 template <typename Raw, typename Piv>
-static bool chunk_maps(int n, int kl, int ku, int u, int U, Raw raw, Piv piv, double* F, double* G) {
-  const int B = kChunk, kuu = kl + ku, WF = B + kl, WB = B + kuu;
-  const int nC = (n + B - 1) / B;
+static bool chunk_maps(int n, int p, int u, int U, Raw raw, Piv piv, double* F, double* G) {
+  const int kl = p, kuu = 2 * p;
   bool ok = true;
-  std::vector<double> X((size_t)WB * WB);
-  for (int c = 0; c < nC; ++c) {
-    const int j0 = c * B;
-    std::fill(X.begin(), X.end(), 0.0);
-    for (int t = 0; t < WF; ++t) X[(size_t)t * WF + t] = 1.0;
+  std::vector<double> X;
+  auto write = [&](bool back, int c, double* out) {
+    const int W = chunk_window(p, back), words = map_words(p, back);
+    const bool two = chunk_tiles(p, back) == 2;
+    double* m = out + ((size_t)c * U + u) * words;
+    for (int i = 0; i < words; ++i) {
+      int t, k;
+      map_entry(i, two, t, k);
+      m[i] = t < W && k < W ? X[(size_t)t * W + k] : 0.0;
+    }
+    if (two)
+      for (int t = 0; t < 16; ++t)
+        for (int k = 16; k < W; ++k) ok = ok && X[(size_t)t * W + k] == 0.0;
+  };
+  for (int c = 0; c < chunk_count(n, p, false); ++c) {
+    const int B = chunk_rows(p, false), W = chunk_window(p, false), j0 = c * B;
+    X.assign((size_t)W * W, 0.0);
+    for (int t = 0; t < W; ++t) X[(size_t)t * W + t] = 1.0;
     for (int j = j0; j < std::min(j0 + B, n - 1); ++j) {
       const int tj = j - j0, tp = piv(j) - j0;
       if (tp != tj)
-        for (int k = 0; k < WF; ++k) std::swap(X[(size_t)tj * WF + k], X[(size_t)tp * WF + k]);
+        for (int k = 0; k < W; ++k) std::swap(X[(size_t)tj * W + k], X[(size_t)tp * W + k]);
       for (int i = 1; i <= kl && j + i < n; ++i) {
-        const double l = raw(kl + ku + i, j);
-        for (int k = 0; k < WF; ++k) X[(size_t)(tj + i) * WF + k] -= l * X[(size_t)tj * WF + k];
+        const double l = raw(kuu + i, j);
+        for (int k = 0; k < W; ++k) X[(size_t)(tj + i) * W + k] -= l * X[(size_t)tj * W + k];
       }
     }
-    for (int k = 0; k < WF; ++k)
-      for (int t = 0; t < WF; ++t) {
-        const double x = X[(size_t)t * WF + k];
-        if (t >= map_lo(k, kl)) F[map_offset(c, k, u, t, kl, WF, U)] = x;
-        else ok = ok && x == 0.0;  // read as the column's zero word
-      }
-    const int T = n - 1 - j0;
-    std::fill(X.begin(), X.end(), 0.0);
-    for (int t = 0; t < WB; ++t) X[(size_t)t * WB + t] = 1.0;
+    write(false, c, F);
+  }
+  for (int c = 0; c < chunk_count(n, p, true); ++c) {
+    const int B = chunk_rows(p, true), W = chunk_window(p, true), T = n - 1 - c * B;
+    X.assign((size_t)W * W, 0.0);
+    for (int t = 0; t < W; ++t) X[(size_t)t * W + t] = 1.0;
     for (int j = T; j > T - B && j >= 0; --j) {
       const int tj = T - j;
-      const double dg = raw(kl + ku, j);
-      for (int k = 0; k < WB; ++k) X[(size_t)tj * WB + k] /= dg;
+      const double dg = raw(kuu, j);
+      for (int k = 0; k < W; ++k) X[(size_t)tj * W + k] /= dg;
       for (int i = 1; i <= kuu && j - i >= 0; ++i) {
-        const double u = raw(kuu - i, j);
-        for (int k = 0; k < WB; ++k) X[(size_t)(tj + i) * WB + k] -= u * X[(size_t)tj * WB + k];
+        const double l = raw(kuu - i, j);
+        for (int k = 0; k < W; ++k) X[(size_t)(tj + i) * W + k] -= l * X[(size_t)tj * W + k];
       }
     }
-    for (int k = 0; k < WB; ++k)
-      for (int t = 0; t < WB; ++t) {
-        const double x = X[(size_t)t * WB + k];
-        if (t >= map_lo(k, 0)) G[map_offset(c, k, u, t, 0, WB, U)] = x;
-        else ok = ok && x == 0.0;
-      }
+    write(true, c, G);
   }
   return ok;
 }
@@ -573,13 +573,15 @@ __global__ void __launch_bounds__(64) k_setup_homog(GpuSetup g) {
 // forward, 1 L_k back, 2 H_k forward, 3 H_k back (chunk_maps' steps).
 __global__ void __launch_bounds__(64) k_setup_maps(GpuSetup g, double* lf, double* lb, double* hf, double* hb) {
 #pragma clang fp contract(off)
-  constexpr int WMAX = kChunk + 16;  // B + 2p for p <= 8
+  constexpr int WMAX = 32;
   __shared__ double X[WMAX * WMAX];
-  const int c = blockIdx.x, u = blockIdx.y, which = blockIdx.z >> 1, back = blockIdx.z & 1;
-  const int lane = threadIdx.x, n = g.n, kl = g.kl, kuu = g.kl + g.ku, B = kChunk;
+  const int c = blockIdx.x, u = blockIdx.y, which = blockIdx.z >> 1;
+  const bool back = blockIdx.z & 1;
+  const int lane = threadIdx.x, n = g.n, kl = g.kl, kuu = g.kl + g.ku;
+  if (c >= chunk_count(n, kl, back)) return;
   const double* ab = g.band + (size_t)(which * g.U + u) * g.rows * n;
   const int* pv = g.piv + (size_t)(which * g.U + u) * n;
-  const int W = back ? B + kuu : B + kl;
+  const int B = chunk_rows(kl, back), W = chunk_window(kl, back);
   for (int e = lane; e < W * W; e += 64) X[e] = (e / W == e % W) ? 1.0 : 0.0;
   __syncthreads();
   const int j0 = c * B;
@@ -621,15 +623,17 @@ __global__ void __launch_bounds__(64) k_setup_maps(GpuSetup g, double* lf, doubl
       __syncthreads();
     }
   }
-  double* F = which == 0 ? (back ? lb : lf) : (back ? hb : hf);
-  const int lag = back ? 0 : kl;
-  bool bad = false;
-  for (int e = lane; e < W * W; e += 64) {
-    const int t = e / W, k = e % W;
-    const double x = X[t * W + k];
-    if (t >= map_lo(k, lag)) F[map_offset(c, k, u, t, lag, W, g.U)] = x;
-    else bad = bad || x != 0.0;
+  const int words = map_words(kl, back);
+  const bool two = chunk_tiles(kl, back) == 2;
+  double* F = (which == 0 ? (back ? lb : lf) : (back ? hb : hf)) + ((size_t)c * g.U + u) * words;
+  for (int i = lane; i < words; i += 64) {
+    int t, k;
+    map_entry(i, two, t, k);
+    F[i] = t < W && k < W ? X[t * W + k] : 0.0;
   }
+  bool bad = false;
+  if (two)
+    for (int e = lane; e < 16 * (W - 16); e += 64) bad = bad || X[(e & 15) * W + 16 + (e >> 4)] != 0.0;
   if (bad) g.flag[1] = 1;
 }
 
@@ -748,6 +752,14 @@ int walls_setup(Ctx* c) {
   build_stencils(y, p, d1, d2);
   if ((rc = upload_vec(c, &t->d1w, d1.w))) return rc;
   if ((rc = upload_vec(c, &t->d1j0, d1.j0))) return rc;
+  auto transposed = [&](const Stencil& d) {
+    std::vector<double> w(d.w.size());
+    for (int i = 0; i < Ny; ++i)
+      for (int k = 0; k < d.width; ++k) w[(size_t)k * Ny + i] = d.w[(size_t)i * d.width + k];
+    return w;
+  };
+  if ((rc = upload_vec(c, &t->d1t, transposed(d1)))) return rc;
+  if ((rc = upload_vec(c, &t->d2t, transposed(d2)))) return rc;
   if ((rc = upload_vec(c, &t->d2w, d2.w))) return rc;
   if ((rc = upload_vec(c, &t->d2j0, d2.j0))) return rc;
   if ((rc = upload_vec(c, &t->qw, quadrature_weights(y, g.ly)))) return rc;
@@ -784,8 +796,8 @@ int walls_setup(Ctx* c) {
   if ((rc = upload_vec(c, &t->umode, umode))) return rc;
   // the chunk maps of the L_k and H_k solves, one per class (not when the
   // sequential sweeps are requested)
-  const int B = kChunk, WF = B + kl, WB = B + kl + ku, nC = (Ny + B - 1) / B;
-  const size_t nf = (size_t)nC * U * map_pre(WF, kl, WF), nb = (size_t)nC * U * map_pre(WB, 0, WB);
+  const size_t nf = (size_t)chunk_count(Ny, p, false) * U * map_words(p, false),
+               nb = (size_t)chunk_count(Ny, p, true) * U * map_words(p, true);
   // the chunked solve also stages three right-hand sides per mode pair in
   // LDS (2 * 3 * (Ny + 32) complex values), which must fit in 64 KiB
   const bool maps_fit = nf < (1ull << 28) && nb < (1ull << 28) &&
@@ -845,13 +857,7 @@ int walls_setup(Ctx* c) {
       for (double** m : {&t->lk_bmap, &t->hk_bmap})
         if (!(*m = static_cast<double*>(c->alloc(nb * sizeof(double)))))
           return c->fail(DNSMI_ENOMEM, "device allocation failed");
-      // each packed column's leading zero word is read, never written
-      if (hipMemset(t->lk_fmap, 0, nf * sizeof(double)) != hipSuccess ||
-          hipMemset(t->hk_fmap, 0, nf * sizeof(double)) != hipSuccess ||
-          hipMemset(t->lk_bmap, 0, nb * sizeof(double)) != hipSuccess ||
-          hipMemset(t->hk_bmap, 0, nb * sizeof(double)) != hipSuccess)
-        return c->fail(DNSMI_EHIP, "memset");
-      hipLaunchKernelGGL(k_setup_maps, dim3(nC, U, 4), dim3(64), 0, nullptr, gs, t->lk_fmap, t->lk_bmap,
+      hipLaunchKernelGGL(k_setup_maps, dim3(std::max(chunk_count(Ny, p, false), chunk_count(Ny, p, true)), U, 4), dim3(64), 0, nullptr, gs, t->lk_fmap, t->lk_bmap,
                          t->hk_fmap, t->hk_bmap);
       if ((rc = check_launch(c, "setup_maps"))) return rc;
     }
@@ -865,7 +871,7 @@ int walls_setup(Ctx* c) {
       return c->fail(DNSMI_EHIP, "set-up: read flags");
     for (void* q : {(void*)k2d, (void*)gs.band, (void*)gs.piv, (void*)gs.flag, (void*)gs.minv}) c->release(q);
     if (flag[0]) return c->fail(DNSMI_ESINGULAR, "banded LU hit a zero pivot");
-    if (flag[1]) return c->fail(DNSMI_EINVAL, "chunk maps: nonzero entry outside the packed region");
+    if (flag[1]) return c->fail(DNSMI_EINVAL, "chunk maps: nonzero entry outside the window's tiles");
   } else {
     std::vector<double> lk_ab((size_t)Ny * rows * M), hk_ab((size_t)Ny * rows * M);
     std::vector<int> lk_piv((size_t)Ny * M), hk_piv((size_t)Ny * M);
@@ -968,8 +974,8 @@ int walls_setup(Ctx* c) {
           auto lpiv = [&](int j) { return lk_piv[(size_t)j * M + m]; };
           auto hraw = [&](int r, int j) { return hk_ab[((size_t)j * rows + r) * M + m]; };
           auto hpiv = [&](int j) { return hk_piv[(size_t)j * M + m]; };
-          const bool a = chunk_maps(Ny, kl, ku, u, U, lraw, lpiv, lf.data(), lb.data());
-          const bool b = chunk_maps(Ny, kl, ku, u, U, hraw, hpiv, hf.data(), hb.data());
+          const bool a = chunk_maps(Ny, p, u, U, lraw, lpiv, lf.data(), lb.data());
+          const bool b = chunk_maps(Ny, p, u, U, hraw, hpiv, hf.data(), hb.data());
           if (!a || !b) ok[w] = 0;
         }
       };
@@ -978,7 +984,7 @@ int walls_setup(Ctx* c) {
       work(0);
       for (auto& th : pool) th.join();
       for (char o : ok)
-        if (!o) return c->fail(DNSMI_EINVAL, "chunk maps: nonzero entry outside the packed region");
+        if (!o) return c->fail(DNSMI_EINVAL, "chunk maps: nonzero entry outside the window's tiles");
       if ((rc = upload_vec(c, &t->lk_fmap, lf))) return rc;
       if ((rc = upload_vec(c, &t->lk_bmap, lb))) return rc;
       if ((rc = upload_vec(c, &t->hk_fmap, hf))) return rc;
@@ -996,14 +1002,20 @@ int walls_setup(Ctx* c) {
   std::snprintf(note, sizeof note, "imm_setup=%s(%.1f ms) curl_rows=%d ", on_gpu ? "gpu" : "host", setup_ms,
                 t->curl_ty);
   if (want_maps) {
-    // the chunked solve's mode order: by map, so that the two modes of a
-    // wavefront share theirs wherever two modes have the same k^2
+    // the chunked solves' items: two modes of one class (one map), the second
+    // marked absent (its complement) where a class's count is odd
     std::vector<int> order(M);
     for (int m = 0; m < M; ++m) order[m] = m;
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return umode[a] < umode[b]; });
-    order.resize((size_t)2 * ((M + 1) / 2), order[M - 1]);  // a spare slot repeats the last mode
-    std::vector<int2> sched(order.size());
-    for (size_t i = 0; i < order.size(); ++i) sched[i] = make_int2(order[i], umode[order[i]]);
+    std::vector<int2> sched;
+    for (int i = 0; i < M;) {
+      const int m = order[i], u = umode[m];
+      const bool two = i + 1 < M && umode[order[i + 1]] == u;
+      sched.push_back(make_int2(m, u));
+      sched.push_back(make_int2(two ? order[i + 1] : ~m, u));
+      i += two ? 2 : 1;
+    }
+    t->items = (int)(sched.size() / 2);
     if ((rc = upload_vec(c, &t->sched, sched))) return rc;
   }
   if ((rc = upload_vec(c, &t->mkx, mkx))) return rc;
@@ -1205,8 +1217,7 @@ struct ImmArgs {
   cx<double>* out;        // velocity_new (may alias uj)
   cx<double>* corr;       // correction (may be null)
   double* partials;       // per-block sum of quadrature-weighted k_metric |delta|^2
-  const double *d1w, *d2w, *qw;
-  const int *d1j0, *d2j0;
+  const double *d1w, *d2w, *qw;  // stencil weights as [k][y]
   const double *lk_ab, *hk_ab;
   const int *lk_piv, *hk_piv;
   const double* vq;    // [map][y][4]: v1, v2, q1, q2
@@ -1236,86 +1247,91 @@ __device__ __forceinline__ cx<double>* svec(const ImmArgs& a, int v, int m) {
 }
 __device__ __forceinline__ cx<double> ikm(double k, cx<double> z) { return {-k * z.y, k * z.x}; }
 
-// D1 / D2 stencils at row y of a row r (global or LDS) whose element y is
-// at r[y * stride]
+// D1 (S = p + 1 points) / D2 (S = p + 2) stencils: row y's weights, and their
+// sum over a row r (global or LDS) whose element y is at r[y * stride].  The
+// first point is build_stencils' j0, computed: a load of it would stand
+// before every stencil's reads.
 template <int S>
-__device__ __forceinline__ cx<double> stencil(const double* w, const int* j0t, const cx<double>* r,
-                                              int y, size_t stride = 1) {
-  cx<double> s{0, 0};
-  const int j0 = j0t[y];
+struct Weights {
+  double w[S];
+  int j0;
+  __device__ __forceinline__ Weights() {}
+  __device__ __forceinline__ Weights(const double* t, int Ny, int y) {
+    j0 = max(0, min(y - S / 2, Ny - S));
 #pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const double wk = w[y * S + k];
-    const cx<double> v = r[(j0 + k) * stride];
-    s.x += wk * v.x;
-    s.y += wk * v.y;
+    for (int k = 0; k < S; ++k) w[k] = t[(size_t)k * Ny + y];
   }
-  return s;
-}
+  __device__ __forceinline__ cx<double> operator()(const cx<double>* r, size_t stride = 1) const {
+    cx<double> s{0, 0};
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      const cx<double> v = r[(j0 + k) * stride];
+      s.x += w[k] * v.x;
+      s.y += w[k] * v.y;
+    }
+    return s;
+  }
+};
 
 // Per-row arithmetic of the parallel phases, shared by the five-launch
-// form and the fused chunked form (so both compute the same values, bit for
-// bit).  `row` = m Ny, `comp` = M Ny; the rows the stencils read are in LDS.
+// form and the fused form (so both compute the same values, bit for bit).
+// `row` = m Ny, `comp` = M Ny; the rows the stencils read are in LDS.
 
-// d_hat^n at row y (phase 1): i kx u_x + D1 u_y + i kz u_z; un1 = u^n_y's row.
+// c N_j + (1 - c) N_n at element e of a field (phases 1 and 3).
+__device__ __forceinline__ cx<double> imm_n_at(const ImmArgs& a, size_t e) {
+  const cx<double> j = a.nj[e], n = a.nn[e];
+  const double g = 1.0 - a.c;
+  return {__builtin_fma(a.c, j.x, g * n.x), __builtin_fma(a.c, j.y, g * n.y)};
+}
+
+// d_hat^n at row y (phase 1): i kx u_x + D1 u_y + i kz u_z; un1 = u^n_y's
+// row, ux and uz the other components there.
 template <int PO>
-__device__ __forceinline__ cx<double> imm_dhat_at(const ImmArgs& a, const cx<double>* un1, size_t row,
-                                                  size_t comp, double kx, double kz, int y) {
-  const cx<double> dv = stencil<PO + 1>(a.d1w, a.d1j0, un1, y);
-  const cx<double> t0 = ikm(kx, a.un[row + y]);
-  const cx<double> t2 = ikm(kz, a.un[2 * comp + row + y]);
+__device__ __forceinline__ cx<double> imm_dhat_at(const Weights<PO + 1>& d1, const cx<double>* un1, cx<double> ux,
+                                                  cx<double> uz, double kx, double kz) {
+  const cx<double> dv = d1(un1);
+  const cx<double> t0 = ikm(kx, ux), t2 = ikm(kz, uz);
   return {(t0.x + dv.x) + t2.x, (t0.y + dv.y) + t2.y};
 }
 
-// f_hat at row y (phase 1), zero on the walls; dh = d_hat^n's row, nj1 and
-// nn1 the y rows of N_j and N_n.
+// f_hat at row y (phase 1), zero on the walls; dh = d_hat^n's row, nc1 the
+// y row of c N_j + (1 - c) N_n, ncx and ncz its other components at y.
 template <int PO>
-__device__ __forceinline__ cx<double> imm_fhat_at(const ImmArgs& a, const cx<double>* dh, const cx<double>* nj1,
-                                                  const cx<double>* nn1, size_t row, size_t comp, double kx,
+__device__ __forceinline__ cx<double> imm_fhat_at(const ImmArgs& a, const Weights<PO + 1>& d1,
+                                                  const Weights<PO + 2>& d2, const cx<double>* dh,
+                                                  const cx<double>* nc1, cx<double> ncx, cx<double> ncz, double kx,
                                                   double kz, double k2, int y) {
-  if (y <= 0 || y >= a.Ny - 1) return {0, 0};
-  constexpr int S1 = PO + 1, S2 = PO + 2;
-  const double dt = a.dt, cc = a.c, nu = a.nu;
+  const bool wall = y <= 0 || y >= a.Ny - 1;
+  const double idt = 1.0 / a.dt, g = (1 - a.c) * a.nu;
   const cx<double> d = dh[y];
-  const cx<double> dvj = stencil<S1>(a.d1w, a.d1j0, nj1, y);
-  const cx<double> dvn = stencil<S1>(a.d1w, a.d1j0, nn1, y);
-  const cx<double> aj = ikm(kx, a.nj[row + y]), cj = ikm(kz, a.nj[2 * comp + row + y]);
-  const cx<double> an = ikm(kx, a.nn[row + y]), cn = ikm(kz, a.nn[2 * comp + row + y]);
-  const cx<double> divj = {(aj.x + dvj.x) + cj.x, (aj.y + dvj.y) + cj.y};
-  const cx<double> divn = {(an.x + dvn.x) + cn.x, (an.y + dvn.y) + cn.y};
-  const cx<double> d2d = stencil<S2>(a.d2w, a.d2j0, dh, y);
+  const cx<double> dv = d1(nc1);
+  const cx<double> t0 = ikm(kx, ncx), t2 = ikm(kz, ncz);
+  const cx<double> dn = {(t0.x + dv.x) + t2.x, (t0.y + dv.y) + t2.y};
+  const cx<double> d2d = d2(dh);
   const cx<double> lkd = {d2d.x - k2 * d.x, d2d.y - k2 * d.y};
-  const double g = (1 - cc) * nu;
-  return {((d.x / dt + cc * divj.x) + (1 - cc) * divn.x) + g * lkd.x,
-          ((d.y / dt + cc * divj.y) + (1 - cc) * divn.y) + g * lkd.y};
+  return wall ? cx<double>{0, 0} : cx<double>{(idt * d.x + dn.x) + g * lkd.x, (idt * d.y + dn.y) + g * lkd.y};
 }
 
 // R_c at row y for the three components (phase 3), zero on the walls; pp =
-// the p_P row, ur = the rows of u^n ([c][Ny]).
+// the p_P row, ur = the rows of u^n (component c at ur + c ld), nc = c N_j +
+// (1 - c) N_n at y.
 template <int PO>
-__device__ __forceinline__ void imm_r_at(const ImmArgs& a, const cx<double>* pp, const cx<double>* ur, size_t row,
-                                         size_t comp, double kx, double kz, double k2, int y,
+__device__ __forceinline__ void imm_r_at(const ImmArgs& a, const Weights<PO + 1>& d1, const Weights<PO + 2>& d2,
+                                         const cx<double>* pp, const cx<double>* ur, int ld,
+                                         const cx<double> (&nc)[3], double kx, double kz, double k2, int y,
                                          cx<double> (&r)[3]) {
-  const int Ny = a.Ny;
-  if (y <= 0 || y >= Ny - 1) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c) r[c] = {0, 0};
-    return;
-  }
-  constexpr int S1 = PO + 1, S2 = PO + 2;
-  const double dt = a.dt, cc = a.c, nu = a.nu;
+  const bool wall = y <= 0 || y >= a.Ny - 1;
+  const double idt = 1.0 / a.dt, g = (1.0 - a.c) * a.nu;
   const cx<double> p = pp[y];
-  const cx<double> dpp[3] = {ikm(kx, p), stencil<S1>(a.d1w, a.d1j0, pp, y), ikm(kz, p)};
+  const cx<double> dpp[3] = {ikm(kx, p), d1(pp), ikm(kz, p)};
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    const cx<double>* unc = ur + c * Ny;
+    const cx<double>* unc = ur + c * ld;
     const cx<double> u = unc[y];
-    const cx<double> du = stencil<S2>(a.d2w, a.d2j0, unc, y);
+    const cx<double> du = d2(unc);
     const cx<double> l = {du.x - k2 * u.x, du.y - k2 * u.y};
-    const double g = (1.0 - cc) * nu;
-    const cx<double> hm = {(1.0 / dt) * u.x + g * l.x, (1.0 / dt) * u.y + g * l.y};
-    const cx<double> Nj = a.nj[c * comp + row + y], Nn = a.nn[c * comp + row + y];
-    r[c] = {((hm.x - dpp[c].x) + cc * Nj.x) + (1 - cc) * Nn.x, ((hm.y - dpp[c].y) + cc * Nj.y) + (1 - cc) * Nn.y};
+    const cx<double> hm = {idt * u.x + g * l.x, idt * u.y + g * l.y};
+    r[c] = wall ? cx<double>{0, 0} : cx<double>{(hm.x - dpp[c].x) + nc[c].x, (hm.y - dpp[c].y) + nc[c].y};
   }
 }
 
@@ -1324,11 +1340,10 @@ __device__ __forceinline__ void imm_r_at(const ImmArgs& a, const cx<double>* pp,
 template <int PO>
 __device__ __forceinline__ void imm_alpha(const ImmArgs& a, int m, const cx<double>* va, size_t vs,
                                           cx<double>& al1, cx<double>& al2) {
-  constexpr int S1 = PO + 1;
   const int Ny = a.Ny;
   const size_t M = a.M;
   const double kx = a.mkx[m], kz = a.mkz[m];
-  cx<double> dw0 = stencil<S1>(a.d1w, a.d1j0, va, 0, vs), dw1 = stencil<S1>(a.d1w, a.d1j0, va, Ny - 1, vs);
+  cx<double> dw0 = Weights<PO + 1>(a.d1w, Ny, 0)(va, vs), dw1 = Weights<PO + 1>(a.d1w, Ny, Ny - 1)(va, vs);
   if (kx * kx + kz * kz == 0.0) dw0 = {0, 0};
   const double m00 = a.minv[0 * M + m], m01 = a.minv[1 * M + m];
   const double m10 = a.minv[2 * M + m], m11 = a.minv[3 * M + m];
@@ -1337,14 +1352,14 @@ __device__ __forceinline__ void imm_alpha(const ImmArgs& a, int m, const cx<doub
 }
 
 // Row y of the assembly (phase 5): the corrected velocity into out (and the
-// correction into corr) when `store`; returns k_metric |delta|^2 of the row
-// (before its quadrature weight).  ua, va, wa: v_arb's rows (stride vs).
+// correction into corr); returns k_metric |delta|^2 of the row (before its
+// quadrature weight).  ua, va, wa: v_arb's rows (stride vs).
 __device__ __forceinline__ double imm_assemble_at(const ImmArgs& a, int m, size_t row, size_t comp, double kx,
-                                                  double kz, const cx<double>* ua, const cx<double>* va,
+                                                  double kz, double4 w, const cx<double> (&uj)[3],
+                                                  const cx<double>* ua, const cx<double>* va,
                                                   const cx<double>* wa, size_t vs, cx<double> al1,
-                                                  cx<double> al2, int y, bool store) {
+                                                  cx<double> al2, int y) {
   const double km = (m % a.Nkx == 0) ? 1.0 : 2.0;
-  const double4 w = reinterpret_cast<const double4*>(a.vq)[(size_t)a.umode[m] * a.Ny + y];
   const double v1 = w.x, v2 = w.y, q1 = w.z, q2 = w.w;
   const cx<double> vv = va[(size_t)y * vs];
   const cx<double> vn = {(vv.x + al1.x * v1) + al2.x * v2, (vv.y + al1.y * v1) + al2.y * v2};
@@ -1356,12 +1371,9 @@ __device__ __forceinline__ double imm_assemble_at(const ImmArgs& a, int m, size_
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     const size_t idx = c * comp + row + y;
-    const cx<double> old = a.uj[idx];
-    const cx<double> d = {nw[c].x - old.x, nw[c].y - old.y};
-    if (store) {
-      a.out[idx] = nw[c];
-      if (a.corr) a.corr[idx] = d;
-    }
+    const cx<double> d = {nw[c].x - uj[c].x, nw[c].y - uj[c].y};
+    a.out[idx] = nw[c];
+    if (a.corr) a.corr[idx] = d;
     s += km * (d.x * d.x) + km * (d.y * d.y);
   }
   return s;
@@ -1372,27 +1384,27 @@ __device__ __forceinline__ double imm_assemble_at(const ImmArgs& a, int m, size_
 template <int PO>
 __global__ void __launch_bounds__(kImmT) k_imm_fhat(ImmArgs a) {
   if (a.act && *a.act == 0) return;
-  // LDS: d_hat, then the y rows of u^n_y, N_j,y and N_n,y (the D1 stencils'
-  // operands, read once from HBM)
+  // LDS: d_hat, then the y rows of u^n and c N_j + (1 - c) N_n (the D1
+  // stencils' operands, read once from HBM)
   extern __shared__ cx<double> dh[];
   const int m = blockIdx.x, Ny = a.Ny;
   const size_t comp = (size_t)a.M * Ny, row = (size_t)m * Ny;
   const double kx = a.mkx[m], kz = a.mkz[m];
   const double k2 = kx * kx + kz * kz;
   cx<double>* un1 = dh + Ny;
-  cx<double>* nj1 = dh + 2 * Ny;
-  cx<double>* nn1 = dh + 3 * Ny;
+  cx<double>* nc1 = dh + 2 * Ny;
   for (int y = threadIdx.x; y < Ny; y += blockDim.x) {
     un1[y] = a.un[comp + row + y];
-    nj1[y] = a.nj[comp + row + y];
-    nn1[y] = a.nn[comp + row + y];
+    nc1[y] = imm_n_at(a, comp + row + y);
   }
   __syncthreads();
-  for (int y = threadIdx.x; y < Ny; y += blockDim.x) dh[y] = imm_dhat_at<PO>(a, un1, row, comp, kx, kz, y);
+  for (int y = threadIdx.x; y < Ny; y += blockDim.x)
+    dh[y] = imm_dhat_at<PO>(Weights<PO + 1>(a.d1w, Ny, y), un1, a.un[row + y], a.un[2 * comp + row + y], kx, kz);
   __syncthreads();
   cx<double>* f = svec(a, V_F, m);
   for (int y = threadIdx.x; y < Ny; y += blockDim.x)
-    f[y * VS] = imm_fhat_at<PO>(a, dh, nj1, nn1, row, comp, kx, kz, k2, y);
+    f[y * VS] = imm_fhat_at<PO>(a, Weights<PO + 1>(a.d1w, Ny, y), Weights<PO + 2>(a.d2w, Ny, y), dh, nc1,
+                                imm_n_at(a, row + y), imm_n_at(a, 2 * comp + row + y), kx, kz, k2, y);
 }
 
 // Phases 2 and 4: solve ab x = rhs per (mode, right-hand side r =
@@ -1515,149 +1527,181 @@ __global__ void __launch_bounds__(kSweepLanes)
 }
 
 // Phases 2 and 4, chunked form: the same solves through the precomputed
-// chunk maps (chunk_maps).  32 lanes per mode, two modes per wavefront;
-// lane t forms output t of each chunk's map from the window, which the
-// mode's lanes share through LDS, so the dependent chain is nC chunks
-// instead of Ny rows, and every load is coalesced and independent of the
-// recurrence.  The right-hand sides are staged in LDS at the start; a
-// chunk's map is loaded S - 1 chunks ahead through S register slots (the
-// chunk loop is unrolled by S so the slots are static).  The forward
-// results stay in LDS for the back substitution.  NR right-hand sides per
-// mode share the maps; the two modes of a wavefront mostly share one map
-// (the modes come in the order `sched`, grouped by k^2), whose words are
-// then fetched once for both.  Lanes in a packed column's structural zeros
-// read its zero word, so the sums are those of the full maps.
+// chunk maps (chunk_maps), on the FP64 matrix cores.  A wavefront takes two
+// modes of one k^2 class: its right-hand sides, real and imaginary parts
+// apart, are the columns of a matrix (4 of 16 for L_k, 12 of 16 for H_k), and
+// a chunk is (map) x (window) in 16-row tiles of v_mfma_f64_16x16x4_f64.  Lane
+// (g = lane / 16, col = lane % 16) holds rows 4 i + g of a tile's result and
+// row 4 q + g of its k step q: a result is the next chunk's operand as it
+// stands, the rows that stay in the window moving by whole registers, so the
+// chain over the chunks never leaves the registers.  Rows entering the window
+// come from the LDS rows the solve works in (in place: a chunk's results
+// overwrite rows that have left the window), and results go back there, off
+// the chain.
+//
+// Bound: the products, 27 ns each and one per SIMD at a time, 128 + 156 of
+// them for a solve at Ny = 256, p = 6 (7.6 us), where broadcasting the window to
+// one lane per map row through LDS took 50 FMA steps behind 150 LDS reads per
+// 16 rows (1.5 us).  Windows of 16 rows (12 to 8 new ones each) take fewer
+// products per row than two-tile ones of 16 new rows (p = 4: 0.83 against
+// 1.25), and operands in load order cost the vector memory path a quarter of
+// what gathering them from packed columns did (25 cycles per load on each CU,
+// four solving wavefronts: 1000 to 1400 cycles per 16 rows, more loads in
+// flight only made it worse).
+typedef double wd4 __attribute__((ext_vector_type(4)));
 
-// Byte offsets of lane t's words in one chunk's maps (the same for every
-// chunk): rows below a column's first stored row read its zero word; lanes
-// past the window read row w-1 and are never stored.  They fit 32 bits
-// (the maps are at most 2^28 words).
-template <int W, int LAG>
-__device__ __forceinline__ void map_offsets(unsigned (&o)[W], int U, int u, int t) {
-  const int tt = t < W ? t : W - 1;
-#pragma unroll
-  for (int k = 0; k < W; ++k) o[k] = 8u * (unsigned)map_word_at(k, u, tt, LAG, W, U);
-}
-
-// Lane t's row of chunk c's map (chunks past the last repeat it): buffer
-// loads from a resource over the chunk's maps (base and size in scalar
-// registers) at the lane's 32-bit offsets.  Flat 64-bit addresses would need
-// a pair of address registers per load, and the compiler, reusing those of
-// loads still in flight, waited for every outstanding load at each chunk
-// step, which undid the prefetch; a buffer load needs none.  Offsets past
-// the chunk's maps (none, by construction) would read zero.
-template <int W, int LAG>
-__device__ __forceinline__ void map_row(double (&f)[W], const double* __restrict__ map,
-                                        const unsigned (&o)[W], int U, int c, int nC) {
-  const int words = U * map_pre(W, LAG, W);
-  const double* base = map + (size_t)(c < nC ? c : nC - 1) * words;
-  const __amdgpu_buffer_rsrc_t r =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(base), 0, words * (int)sizeof(double), 0x00020000);
-#pragma unroll
-  for (int k = 0; k < W; ++k)
-    f[k] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)o[k], 0, 0));
-}
-
-// acc[r] += sum_k map[t][k] win[r][k] in order k = 0, 1, ...; the window
-// words are read from LDS in batches of KB before their products, so that
-// a batch's reads are in flight together.
-template <int W, int NR, int KB>
-__device__ __forceinline__ void window_dot(cx<double> (&acc)[NR], const double (&f)[W],
-                                           const cx<double>* win) {
-#pragma unroll
-  for (int k0 = 0; k0 < W; k0 += KB) {
-    cx<double> w[KB][NR];
-#pragma unroll
-    for (int kk = 0; kk < KB; ++kk)
-#pragma unroll
-      for (int r = 0; r < NR; ++r)
-        if (k0 + kk < W) w[kk][r] = win[r * 32 + k0 + kk];
-#pragma unroll
-    for (int kk = 0; kk < KB; ++kk) {
-      if (k0 + kk >= W) break;
-      const double fk = f[k0 + kk];
-#pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        acc[r].x += fk * w[kk][r].x;
-        acc[r].y += fk * w[kk][r].y;
-      }
-    }
-  }
-}
-
-// The window is shared by the mode's lanes, all in this wavefront, whose
-// LDS operations complete in issue order.
+// The LDS rows of a solve belong to one wavefront, whose LDS operations
+// complete in issue order.
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
 
-// One forward chunk: window position t <-> row cB + t.  vec holds the
-// right-hand sides (row stride 1, Ny rows each); the chunk overwrites rows
-// below (c + 1) B with results and reads rows from (c + 1) B + KL on.  pf
-// receives the map of chunk c + S - 1.
-template <int PO, int NR, int S>
-__device__ __forceinline__ void fwd_chunk(const double (&f)[kChunk + PO], double (&pf)[kChunk + PO],
-                                          const double* __restrict__ fmap,
-                                          const unsigned (&o)[kChunk + PO], int U, cx<double>* vec, cx<double>* win, int t, int c, int nC,
-                                          int Ny) {
-  constexpr int KL = PO, B = kChunk, WF = B + KL;
-  const int frow = (c + 1) * B + t;
-  const bool fr = t >= KL && t < WF && frow < Ny;
-  cx<double> fresh[NR];
-#pragma unroll
-  for (int r = 0; r < NR; ++r) fresh[r] = fr ? vec[r * Ny + frow] : cx<double>{0, 0};
-  map_row<WF, KL>(pf, fmap, o, U, c + S - 1, nC);
-  cx<double> acc[NR];
-#pragma unroll
-  for (int r = 0; r < NR; ++r) acc[r] = cx<double>{0, 0};
-  window_dot<WF, NR, window_batch(PO, NR)>(acc, f, win);
-  wave_sync();
-  const int row = c * B + t;
-#pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    if (t < B && row < Ny) vec[r * Ny + row] = acc[r];
-    if (t >= B && t < WF) win[r * 32 + t - B] = acc[r];
-    if (t >= KL && t < WF) win[r * 32 + t] = fresh[r];
-  }
-  wave_sync();
+// LDS vectors of a solve: Ny rows each between zero rows, so that a window
+// that reaches past either end reads zeros without a test: as many as the last
+// chunk's window has behind its direction's end, the next vector's first ones
+// serving the one before.  Vector v starts at v ld + pad; ld = 4 mod 16 keeps
+// the columns of a wavefront's reads (four rows of each) on different banks.
+__host__ __device__ inline int chunk_pad(int Ny, int p) {
+  const int f = 16 * chunk_tiles(p, false) - 1 - (Ny - 1) % chunk_rows(p, false);
+  const int b = 16 * chunk_tiles(p, true) - 1 - (Ny - 1) % chunk_rows(p, true);
+  return f > b ? f : b;
+}
+__host__ __device__ inline int chunk_ld(int Ny, int p) { return (Ny + chunk_pad(Ny, p) + 11) / 16 * 16 + 4; }
+__host__ __device__ inline int chunk_lds(int Ny, int p, int vectors) {
+  return vectors * chunk_ld(Ny, p) + chunk_pad(Ny, p);
+}
+// Zeros over all rows that are no vector's.
+__device__ __forceinline__ void chunk_zero(cx<double>* lds, int Ny, int p, int vectors) {
+  const int pad = chunk_pad(Ny, p), gap = chunk_ld(Ny, p) - Ny;
+  for (int v = 0; v < vectors; ++v)
+    for (int i = threadIdx.x; i < gap; i += blockDim.x) {
+      const int row = v * chunk_ld(Ny, p) + (i < pad ? i : Ny + i);
+      lds[row] = cx<double>{0, 0};
+    }
+  for (int i = threadIdx.x; i < pad; i += blockDim.x) lds[vectors * chunk_ld(Ny, p) + i] = cx<double>{0, 0};
 }
 
-// One back chunk: window position t <-> row T - t, T = Ny - 1 - cB; pg
-// receives the map of chunk c + S - 1.
-template <int PO, int NR, int S>
-__device__ __forceinline__ void back_chunk(const double (&g)[kChunk + 2 * PO],
-                                           double (&pg)[kChunk + 2 * PO],
-                                           const double* __restrict__ bmap,
-                                           const unsigned (&o)[kChunk + 2 * PO], int U,
-                                           cx<double>* __restrict__ out, size_t vs, bool live,
-                                           cx<double>* vec, cx<double>* win, int t, int c, int nC,
-                                           int Ny) {
-  constexpr int KUU = 2 * PO, B = kChunk, WB = B + KUU;
-  map_row<WB, 0>(pg, bmap, o, U, c + S - 1, nC);
-  const int T = Ny - 1 - c * B;
-  const int frow = T - B - t;
-  const bool fr = t >= KUU && t < WB && frow >= 0;
-  cx<double> fresh[NR];
+// Chunk c's operands e, e + 1 of this lane (chunks past the last repeat it).
+struct MapChunk {
+  const double2* p;
+  __device__ __forceinline__ MapChunk(const double* __restrict__ map, int U, int u, int words, int c, int nC, int lane)
+      : p(reinterpret_cast<const double2*>(map + ((size_t)(c < nC ? c : nC - 1) * U + u) * words) + lane) {}
+  __device__ __forceinline__ double2 operator()(int pair) const { return p[pair * 64]; }
+};
+
+// Chunks of maps in registers, loaded that many less one ahead: eight words a
+// lane each in one-tile windows, 24 in two-tile ones.
+template <int PO, bool BACK>
+struct ChunkMaps {
+  static constexpr int R = chunk_tiles(PO, BACK) == 1 ? 4 : 3, N = map_operands(PO, BACK);
+  double f[R][N];
+  // the first R - 1 chunks'
+  __device__ __forceinline__ void start(const double* __restrict__ map, int U, int u, int lane, int Ny) {
 #pragma unroll
-  for (int r = 0; r < NR; ++r) fresh[r] = fr ? vec[r * Ny + frow] : cx<double>{0, 0};
-  cx<double> acc[NR];
+    for (int q = 0; q < R - 1; ++q) {
+      const MapChunk m(map, U, u, map_words(PO, BACK), q, chunk_count(Ny, PO, BACK), lane);
 #pragma unroll
-  for (int r = 0; r < NR; ++r) acc[r] = cx<double>{0, 0};
-  window_dot<WB, NR, window_batch(PO, NR)>(acc, g, win);
-  wave_sync();
-  const int row = T - t;
-#pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    if (t < B && row >= 0 && live) out[r * vs + row] = acc[r];
-    if (t >= B && t < WB) win[r * 32 + t - B] = acc[r];
-    if (t >= KUU && t < WB) win[r * 32 + t] = fresh[r];
+      for (int e = 0; e < N / 2; ++e) {
+        const double2 v = m(e);
+        f[q][2 * e] = v.x;
+        f[q][2 * e + 1] = v.y;
+      }
+    }
   }
+};
+
+// The chunks of one direction.  Window position t <-> row o + s t (o the
+// chunk's first row, s = 1 forward, -1 back), the last KEEP rows stay in the
+// window from one chunk to the next.  pc: the lane's column (element y at
+// pc[2 y]: one part of a complex row); lanes past the columns repeat one, and
+// store its values again.  Window rows are read one chunk ahead, a chunk's
+// results stored one behind.
+//
+// The k steps of rows that were in LDS come first in each sum, those of the
+// rows kept from the chunk before last, and a second tile (whose rows are the
+// kept ones) before the first: a result's latency passes behind products that
+// do not need it.  Behind each product (64 cycles of the matrix core) stands
+// its share of the loads and stores, pinned there: in front of the products
+// they cost half as much again.
+template <int PO, bool BACK>
+__device__ __forceinline__ void chunk_chain(const double* __restrict__ map, int U, int u, int lane, int Ny, double* pc,
+                                            ChunkMaps<PO, BACK>& maps) {
+  constexpr int TILES = chunk_tiles(PO, BACK), B = chunk_rows(PO, BACK), KEEP = BACK ? 2 * PO : PO;
+  constexpr int R = ChunkMaps<PO, BACK>::R, N = ChunkMaps<PO, BACK>::N;
+  constexpr int WR = 4 * TILES, KR = (KEEP + 3) / 4, BR = B / 4, S = BACK ? -1 : 1;
+  static_assert(KR + BR == WR, "kept and new rows fill the window's registers");
+  const int g = lane >> 4, nC = chunk_count(Ny, PO, BACK);
+  double* pg = pc + 2 * ((BACK ? Ny - 1 : 0) + S * g);  // this lane group's row of the first chunk
+  double w[WR], done[BR];                               // the window; chunk c - 1's results
+#pragma unroll
+  for (int i = 0; i < WR; ++i) w[i] = pg[2 * S * 4 * i];
+#pragma unroll
+  for (int i = 0; i < BR; ++i) done[i] = 0.0;
+  auto step = [&](int c, double(&fc)[N], double(&pf)[N]) {
+    const MapChunk m(map, U, u, map_words(PO, BACK), c + R - 1, nC, lane);
+    // (the last chunk asks for its own rows again; chunk 0 stores zeros over
+    // rows that the window holds and chunk 1 stores)
+    double* in = pg + 2 * S * min(c + 1, nC - 1) * B;
+    double* out = pg + 2 * S * max(c - 1, 0) * B;
+    double fresh[WR];
+    wd4 acc[TILES];
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) acc[i] = wd4{0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      // product e: tile, k step q, operand of the map
+      const int tile = TILES == 1 || e >= 8 ? 0 : 1, K = TILES == 1 || e >= 8 ? 4 : 8;
+      const int i = TILES == 2 && e >= 8 ? e - 8 : e, kr = KR < K ? KR : 0, q = i < K - kr ? kr + i : i - (K - kr);
+      acc[tile] = __builtin_amdgcn_mfma_f64_16x16x4f64(fc[TILES == 2 && e >= 8 ? 8 + q : q], w[q], acc[tile], 0, 0, 0);
+      if (e < N / 2) {
+        const double2 v = m(e);
+        pf[2 * e] = v.x;
+        pf[2 * e + 1] = v.y;
+      }
+      if (e < BR) out[2 * S * 4 * e] = done[e < BR ? e : 0];
+      if (KR + e < WR) fresh[KR + e < WR ? KR + e : 0] = in[2 * S * 4 * (KR + e)];
+      if (e == 0 && KEEP % 4 != 0) fresh[KR - 1] = in[2 * S * 4 * (KR - 1)];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < BR; ++i) done[i] = acc[i >> 2][i & 3];
+#pragma unroll
+    for (int i = 0; i < WR; ++i) {
+      const int o = i + BR < WR ? i + BR : 0;
+      const double kept = acc[o >> 2][o & 3];
+      w[i] = 4 * i + 4 <= KEEP ? kept : 4 * i >= KEEP ? fresh[i] : (4 * i + g < KEEP ? kept : fresh[i]);
+    }
+  };
+  int c = 0;
+  for (; c + R <= nC; c += R) {
+#pragma unroll
+    for (int q = 0; q < R; ++q) step(c + q, maps.f[q], maps.f[(q + R - 1) % R]);
+  }
+#pragma unroll
+  for (int q = 0; q < R - 1; ++q)
+    if (c + q < nC) step(c + q, maps.f[q], maps.f[(q + R - 1) % R]);
+#pragma unroll
+  for (int i = 0; i < BR; ++i)
+    if ((nC - 1) * B + 4 * i + g < Ny) pg[2 * S * ((nC - 1) * B + 4 * i)] = done[i];
+}
+
+// Band solve of this wavefront's columns, in place; maps: the forward maps,
+// started.
+template <int PO>
+__device__ __forceinline__ void chunk_solve(const double* __restrict__ fmap, const double* __restrict__ bmap, int U,
+                                            int u, int lane, int Ny, double* pc, ChunkMaps<PO, false>& maps) {
+  ChunkMaps<PO, true> back;
+  back.start(bmap, U, u, lane, Ny);
+  wave_sync();
+  chunk_chain<PO, false>(fmap, U, u, lane, Ny, pc, maps);
+  wave_sync();
+  chunk_chain<PO, true>(bmap, U, u, lane, Ny, pc, back);
   wave_sync();
 }
 
 // A launch's workgroups go to the 8 XCDs (each with its own L2) in turn:
-// renumbered so that each XCD takes one contiguous range of slots, where
+// renumbered so that each XCD takes one contiguous range of items, where
 // neighbouring modes (grouped by k^2) share chunk-map cache lines.
 __device__ __forceinline__ int xcd_block(int b, int G) {
   constexpr int X = 8;
@@ -1665,236 +1709,216 @@ __device__ __forceinline__ int xcd_block(int b, int G) {
   return x * q + (x < r ? x : r) + i;
 }
 
-template <int PO, int NR, int S>
-__global__ void __launch_bounds__(64, chunk_waves(PO, NR))
+// The lane's column of a solve with NR right-hand sides per mode: modes at
+// sh + half hs, right-hand sides ld apart, real and imaginary part.
+template <int NR>
+__device__ __forceinline__ double* chunk_column(cx<double>* sh, int hs, int ld, int lane) {
+  const int v = min((lane & 15) >> 1, 2 * NR - 1);
+  return reinterpret_cast<double*>(sh + (v / NR) * hs + (v % NR) * ld) + (lane & 1);
+}
+
+// The item's two modes come as (mode, map), the second (a class with an odd
+// count) perhaps marked absent: then it repeats the first and stores nothing.
+__device__ __forceinline__ int2 sched_mode(const int2* __restrict__ sched, int slot, bool& live) {
+  int2 mu = sched[slot];
+  live = mu.x >= 0;
+  if (!live) mu.x = ~mu.x;
+  return mu;
+}
+
+template <int PO, int NR>
+__global__ void __launch_bounds__(64, 2)
     k_band_chunks(ImmArgs a, const double* __restrict__ fmap, const double* __restrict__ bmap,
                   const int2* __restrict__ sched, int U, int vin, int vout) {
   if (a.act && *a.act == 0) return;
-  constexpr int KL = PO, KUU = 2 * PO, B = kChunk, WF = B + KL, WB = B + KUU;
-  static_assert(WB <= 32, "a window fits the 32 lanes of a mode");
-  static_assert(S >= 2, "a map slot in use and at least one being filled");
-  extern __shared__ cx<double> sh[];  // [2][NR][Ny] vectors, then [2][NR][32] windows
-  const int Ny = a.Ny, M = a.M, nC = (Ny + B - 1) / B;
-  const int lane = threadIdx.x, half = lane >> 5, t = lane & 31;
-  const int slot = xcd_block(blockIdx.x, gridDim.x) * 2 + half;
-  const bool live = slot < M;  // a spare half repeats the last mode and stores nothing
-  const int2 mu = sched[slot];
-  const int m = mu.x, u = mu.y;
-  cx<double>* vec = sh + (size_t)half * NR * Ny;
-  cx<double>* win = sh + (size_t)2 * NR * Ny + (size_t)half * NR * 32;
+  extern __shared__ cx<double> lds[];  // chunk_lds(Ny, PO, 2 NR): [2][NR][ld]
+  const int Ny = a.Ny, M = a.M, ld = chunk_ld(Ny, PO), lane = threadIdx.x;
+  cx<double>* sh = lds + chunk_pad(Ny, PO);
+  const int item = xcd_block(blockIdx.x, gridDim.x);
   const size_t vs = (size_t)M * Ny;  // between work vectors (VS = 1: rows contiguous)
-  const cx<double>* __restrict__ rin = a.scratch + ((size_t)vin * M + m) * Ny;
-  cx<double>* __restrict__ out = a.scratch + ((size_t)vout * M + m) * Ny;
-  // the first maps' loads, then the right-hand sides' to LDS (no global
-  // load on the chunk chain), eight rows per lane in flight at a time, all
-  // under one wait; lanes past the last row load and store that row again
-  // (the same value), so nothing branches
-  double f[S][WF];
-  unsigned of[WF];
-  map_offsets<WF, KL>(of, U, u, t);
+  bool live[2];
+  int2 mu[2];
+  for (int h = 0; h < 2; ++h) mu[h] = sched_mode(sched, 2 * item + h, live[h]);
+  ChunkMaps<PO, false> maps;
+  maps.start(fmap, U, mu[0].y, lane, Ny);
+  chunk_zero(lds, Ny, PO, 2 * NR);
+  // the right-hand sides, all in flight (rows past the end load and store the
+  // last one again)
+  for (int i0 = 0; i0 < Ny; i0 += 4 * 64) {
+    cx<double> v[4][2 * NR];
 #pragma unroll
-  for (int q = 0; q < S - 1; ++q) map_row<WF, KL>(f[q], fmap, of, U, q, nC);
-  for (int i0 = 0; i0 < Ny; i0 += 8 * 32) {
-    cx<double> v[8][NR];
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int i = min(i0 + q * 32 + t, Ny - 1);
+      for (int r = 0; r < 2 * NR; ++r)
+        v[q][r] = a.scratch[((size_t)vin * M + mu[r / NR].x) * Ny + (r % NR) * vs + min(i0 + q * 64 + lane, Ny - 1)];
 #pragma unroll
-      for (int r = 0; r < NR; ++r) v[q][r] = rin[r * vs + i];
-    }
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int i = min(i0 + q * 32 + t, Ny - 1);
-#pragma unroll
-      for (int r = 0; r < NR; ++r) vec[r * Ny + i] = v[q][r];
-    }
+      for (int r = 0; r < 2 * NR; ++r) sh[r * ld + min(i0 + q * 64 + lane, Ny - 1)] = v[q][r];
   }
-  {
-    wave_sync();
-    if (t < WF) {
+  chunk_solve<PO>(fmap, bmap, U, mu[0].y, lane, Ny, chunk_column<NR>(sh, NR * ld, ld, lane), maps);
+  for (int i = lane; i < Ny; i += 64)
 #pragma unroll
-      for (int r = 0; r < NR; ++r) win[r * 32 + t] = t < Ny ? vec[r * Ny + t] : cx<double>{0, 0};
-    }
-    wave_sync();
-    for (int c = 0; c < nC; c += S) {
-#pragma unroll
-      for (int q = 0; q < S; ++q) {
-        if (c + q >= nC) break;
-        fwd_chunk<PO, NR, S>(f[q], f[(q + S - 1) % S], fmap, of, U, vec, win, t, c + q, nC, Ny);
-      }
-    }
-  }
-  {
-    double g[S][WB];
-    unsigned og[WB];
-    map_offsets<WB, 0>(og, U, u, t);
-#pragma unroll
-    for (int q = 0; q < S - 1; ++q) map_row<WB, 0>(g[q], bmap, og, U, q, nC);
-    if (t < WB) {
-#pragma unroll
-      for (int r = 0; r < NR; ++r)
-        win[r * 32 + t] = (Ny - 1 - t >= 0) ? vec[r * Ny + Ny - 1 - t] : cx<double>{0, 0};
-    }
-    wave_sync();
-    for (int c = 0; c < nC; c += S) {
-#pragma unroll
-      for (int q = 0; q < S; ++q) {
-        if (c + q >= nC) break;
-        back_chunk<PO, NR, S>(g[q], g[(q + S - 1) % S], bmap, og, U, out, vs, live, vec, win, t,
-                              c + q, nC, Ny);
-      }
-    }
-  }
+    for (int r = 0; r < 2 * NR; ++r)
+      if (live[r / NR]) a.scratch[((size_t)vout * M + mu[r / NR].x) * Ny + (r % NR) * vs + i] = sh[r * ld + i];
 }
 
-// Fused chunked form: two launches per influence-matrix step instead of
-// five.  Phases 1 and 2 (k_imm_lsolve): each mode's f_hat is formed by its
-// 32 lanes straight into the LDS row the chunked L_k solve starts from; the
-// solution p_P goes to V_P.  Phases 3 to 5 (k_imm_hsolve): R_c for the three
-// components straight into LDS, the H_k solve with its results kept in
-// LDS, then alpha and the assembly.  The per-row arithmetic and the chunk
-// chains are those of the five-launch form (same values, bit for bit); only
-// the work vectors' round trips through memory and three launches go.  The
-// forward and back chunk loops are those of k_band_chunks.
-template <int PO, int NR, int S>
-__device__ __forceinline__ void chunk_solve(const double* __restrict__ fmap, const double* __restrict__ bmap,
-                                            int U, int u, int t, int nC, int Ny, cx<double>* vec, cx<double>* win,
-                                            double (&f)[S][kChunk + PO], const unsigned (&of)[kChunk + PO],
-                                            cx<double>* __restrict__ out, size_t vs, bool live) {
-  constexpr int KL = PO, KUU = 2 * PO, B = kChunk, WF = B + KL, WB = B + KUU;
-  wave_sync();
-  if (t < WF) {
-#pragma unroll
-    for (int r = 0; r < NR; ++r) win[r * 32 + t] = t < Ny ? vec[r * Ny + t] : cx<double>{0, 0};
-  }
-  wave_sync();
-  for (int c = 0; c < nC; c += S) {
-#pragma unroll
-    for (int q = 0; q < S; ++q) {
-      if (c + q >= nC) break;
-      fwd_chunk<PO, NR, S>(f[q], f[(q + S - 1) % S], fmap, of, U, vec, win, t, c + q, nC, Ny);
-    }
-  }
-  double g[S][WB];
-  unsigned og[WB];
-  map_offsets<WB, 0>(og, U, u, t);
-#pragma unroll
-  for (int q = 0; q < S - 1; ++q) map_row<WB, 0>(g[q], bmap, og, U, q, nC);
-  if (t < WB) {
-#pragma unroll
-    for (int r = 0; r < NR; ++r) win[r * 32 + t] = (Ny - 1 - t >= 0) ? vec[r * Ny + Ny - 1 - t] : cx<double>{0, 0};
-  }
-  wave_sync();
-  for (int c = 0; c < nC; c += S) {
-#pragma unroll
-    for (int q = 0; q < S; ++q) {
-      if (c + q >= nC) break;
-      back_chunk<PO, NR, S>(g[q], g[(q + S - 1) % S], bmap, og, U, out, vs, live, vec, win, t, c + q, nC, Ny);
-    }
-  }
-}
+// The whole influence-matrix step of two modes of one k^2 class in one
+// workgroup, two wavefronts: everything between the fields and the new
+// velocity stays in four LDS rows per mode and in registers.  Each wavefront
+// does the parallel phases of its mode (lanes along y, YP points each, whose
+// u^n_x, u^n_z and c N_j + (1 - c) N_n wait in registers through the L_k
+// solve: the fields are read once); one of them the solves of both.  The
+// per-row arithmetic and the solves are those of the five-launch form (same
+// values, bit for bit); eight work vectors' round trips through memory and
+// four launches go.
+//
+// Traffic: 15 vector components, and a class's maps for every two modes (860
+// bytes per point at p = 6: more than the fields).  The maps' way from the
+// caches is the bound, not the products, which would take 20 us per item at
+// Ny = 256, p = 6; four items per CU (36 KB of LDS, 256 registers) put one
+// solving wavefront on each SIMD (the first wavefronts of a CU's workgroups
+// start on different ones).  One predictor, with the sequence of launches that
+// was the fastest before: 128 x 256 x 128, p = 6, five launches 623 us, so
+// 296 us; 64 x 128 x 64, p = 4, two launches (solve and parallel phases by
+// each wavefront) 68 us, so 27 us; 48 x 65 x 32, p = 4: 35 us, so 12 us.
+constexpr int kImmRows = 4;       // LDS rows per mode
+constexpr int kImmFusedNy = 278;  // largest Ny of the fused form
 
-// LDS words (complex) per workgroup of the fused kernels
-__host__ __device__ constexpr size_t imm_lsolve_lds(int Ny) { return 2 * ((size_t)5 * Ny + 32); }
-__host__ __device__ constexpr size_t imm_hsolve_lds(int Ny) { return 2 * ((size_t)7 * Ny + 96); }
-
-template <int PO, int S>
-__global__ void __launch_bounds__(64, chunk_waves(PO, 1))
-    k_imm_lsolve(ImmArgs a, const double* __restrict__ fmap, const double* __restrict__ bmap,
-                 const int2* __restrict__ sched, int U) {
+template <int PO, int YP>
+__global__ void __launch_bounds__(128, 2)
+    k_imm_fused(ImmArgs a, const double* __restrict__ lf, const double* __restrict__ lb,
+                const double* __restrict__ hf, const double* __restrict__ hb, const int2* __restrict__ sched, int U) {
   if (a.act && *a.act == 0) return;
-  constexpr int KL = PO, WF = kChunk + KL;
-  // per half: the solve's vector [Ny], its window [32], then d_hat and the
-  // y rows of u^n_y, N_j,y, N_n,y [4][Ny]
-  extern __shared__ cx<double> sh[];
-  const int Ny = a.Ny, M = a.M, nC = (Ny + kChunk - 1) / kChunk;
-  const int lane = threadIdx.x, half = lane >> 5, t = lane & 31;
-  const int slot = xcd_block(blockIdx.x, gridDim.x) * 2 + half;
-  const bool live = slot < M;  // a spare half repeats the last mode and stores nothing
-  const int2 mu = sched[slot];
-  const int m = mu.x, u = mu.y;
-  cx<double>* vec = sh + (size_t)half * Ny;
-  cx<double>* win = sh + (size_t)2 * Ny + (size_t)half * 32;
-  cx<double>* dh = sh + (size_t)2 * Ny + 64 + (size_t)half * 4 * Ny;
-  cx<double>* un1 = dh + Ny;
-  cx<double>* nj1 = dh + 2 * Ny;
-  cx<double>* nn1 = dh + 3 * Ny;
-  // the first maps' loads, then the right-hand side
-  double f[S][WF];
-  unsigned of[WF];
-  map_offsets<WF, KL>(of, U, u, t);
-#pragma unroll
-  for (int q = 0; q < S - 1; ++q) map_row<WF, KL>(f[q], fmap, of, U, q, nC);
+  extern __shared__ cx<double> lds[];  // chunk_lds(Ny, PO, 2 kImmRows): [2][kImmRows][ld]
+  const int Ny = a.Ny, M = a.M, ld = chunk_ld(Ny, PO), hs = kImmRows * ld;
+  cx<double>* sh = lds + chunk_pad(Ny, PO);
+  const int lane = threadIdx.x & 63, half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int item = xcd_block(blockIdx.x, gridDim.x);
+  const bool solver = half == 0;
+  bool live;
+  const int2 mu = sched_mode(sched, 2 * item + half, live);
+  const int m = mu.x, u = __builtin_amdgcn_readfirstlane(mu.y);
+  ChunkMaps<PO, false> maps;
+  if (solver) maps.start(lf, U, u, lane, Ny);
+  chunk_zero(lds, Ny, PO, 2 * kImmRows);
+  cx<double>* r0 = sh + half * hs;
+  cx<double>*r1 = r0 + ld, *r2 = r0 + 2 * ld, *r3 = r0 + 3 * ld;
   const size_t comp = (size_t)M * Ny, row = (size_t)m * Ny;
   const double kx = a.mkx[m], kz = a.mkz[m];
   const double k2 = kx * kx + kz * kz;
-  for (int y = t; y < Ny; y += 32) {
-    un1[y] = a.un[comp + row + y];
-    nj1[y] = a.nj[comp + row + y];
-    nn1[y] = a.nn[comp + row + y];
+  // phase 1: u^n_y in r1, c N_j + (1 - c) N_n (y) in r0, d_hat in r2, f_hat in r3
+  cx<double> ux[YP], uz[YP], nc[YP][3];
+#pragma unroll
+  for (int j = 0; j < YP; ++j) {
+    const int y = min(lane + 64 * j, Ny - 1);
+    ux[j] = a.un[row + y];
+    uz[j] = a.un[2 * comp + row + y];
+    r1[y] = a.un[comp + row + y];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) nc[j][c] = imm_n_at(a, c * comp + row + y);
+    r0[y] = nc[j][1];
+  }
+  // weights of G rows at a time: all their loads in flight, within the registers
+  constexpr int G = YP < 2 ? YP : 2;
+  wave_sync();
+#pragma unroll
+  for (int j0 = 0; j0 < YP; j0 += G) {
+    Weights<PO + 1> d1[G];
+#pragma unroll
+    for (int j = 0; j < G && j0 + j < YP; ++j) d1[j] = Weights<PO + 1>(a.d1w, Ny, min(lane + 64 * (j0 + j), Ny - 1));
+#pragma unroll
+    for (int j = 0; j < G && j0 + j < YP; ++j)
+      r2[min(lane + 64 * (j0 + j), Ny - 1)] = imm_dhat_at<PO>(d1[j], r1, ux[j0 + j], uz[j0 + j], kx, kz);
+    __builtin_amdgcn_sched_barrier(0);
   }
   wave_sync();
-  for (int y = t; y < Ny; y += 32) dh[y] = imm_dhat_at<PO>(a, un1, row, comp, kx, kz, y);
-  wave_sync();
-  for (int y = t; y < Ny; y += 32) vec[y] = imm_fhat_at<PO>(a, dh, nj1, nn1, row, comp, kx, kz, k2, y);
-  chunk_solve<PO, 1, S>(fmap, bmap, U, u, t, nC, Ny, vec, win, f, of, a.scratch + ((size_t)V_P * M + m) * Ny,
-                        (size_t)M * Ny, live);
-}
-
-template <int PO, int S>
-__global__ void __launch_bounds__(64, chunk_waves(PO, 3))
-    k_imm_hsolve(ImmArgs a, const double* __restrict__ fmap, const double* __restrict__ bmap,
-                 const int2* __restrict__ sched, int U) {
-  if (a.act && *a.act == 0) return;
-  constexpr int KL = PO, WF = kChunk + KL;
-  // per half: the solve's vectors [3][Ny], windows [3][32], then the p_P
-  // row and the rows of u^n [4][Ny], whose place the solutions take
-  extern __shared__ cx<double> sh[];
-  const int Ny = a.Ny, M = a.M, nC = (Ny + kChunk - 1) / kChunk;
-  const int lane = threadIdx.x, half = lane >> 5, t = lane & 31;
-  const int slot = xcd_block(blockIdx.x, gridDim.x) * 2 + half;
-  const bool live = slot < M;
-  const int2 mu = sched[slot];
-  const int m = mu.x, u = mu.y;
-  cx<double>* vec = sh + (size_t)half * 3 * Ny;
-  cx<double>* win = sh + (size_t)6 * Ny + (size_t)half * 96;
-  cx<double>* pp = sh + (size_t)6 * Ny + 192 + (size_t)half * 4 * Ny;
-  cx<double>* ur = pp + Ny;
-  double f[S][WF];
-  unsigned of[WF];
-  map_offsets<WF, KL>(of, U, u, t);
 #pragma unroll
-  for (int q = 0; q < S - 1; ++q) map_row<WF, KL>(f[q], fmap, of, U, q, nC);
-  const size_t comp = (size_t)M * Ny, row = (size_t)m * Ny;
-  const double kx = a.mkx[m], kz = a.mkz[m];
-  const double k2 = kx * kx + kz * kz;
-  const cx<double>* P = a.scratch + ((size_t)V_P * M + m) * Ny;
-  for (int y = t; y < Ny; y += 32) {
-    pp[y] = P[y];
+  for (int j0 = 0; j0 < YP; j0 += G) {
+    Weights<PO + 1> d1[G];
+    Weights<PO + 2> d2[G];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) ur[c * Ny + y] = a.un[c * comp + row + y];
+    for (int j = 0; j < G && j0 + j < YP; ++j) {
+      int y = min(lane + 64 * (j0 + j), Ny - 1);
+      if (YP > G) y = opaque(y);
+      d1[j] = Weights<PO + 1>(a.d1w, Ny, y);
+      d2[j] = Weights<PO + 2>(a.d2w, Ny, y);
+    }
+#pragma unroll
+    for (int j = 0; j < G && j0 + j < YP; ++j) {
+      const int y = min(lane + 64 * (j0 + j), Ny - 1);
+      r3[y] = imm_fhat_at<PO>(a, d1[j], d2[j], r2, r0, nc[j0 + j][0], nc[j0 + j][2], kx, kz, k2, y);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
   wave_sync();
-  for (int y = t; y < Ny; y += 32) {
-    cx<double> r[3];
-    imm_r_at<PO>(a, pp, ur, row, comp, kx, kz, k2, y, r);
+  // u^n's rows in r0, r1, r2 (phase 1's other rows are read)
 #pragma unroll
-    for (int c = 0; c < 3; ++c) vec[c * Ny + y] = r[c];
+  for (int j = 0; j < YP; ++j) {
+    const int y = min(lane + 64 * j, Ny - 1);
+    r0[y] = ux[j];
+    r2[y] = uz[j];
   }
-  // the solutions overwrite the p_P row and the u^n rows, read above
-  // before the solve's first wave_sync
-  cx<double>* sol = pp;
-  chunk_solve<PO, 3, S>(fmap, bmap, U, u, t, nC, Ny, vec, win, f, of, sol, (size_t)Ny, true);
-  wave_sync();
+  __syncthreads();
+  // phase 2: p_P in r3
+  if (solver) {
+    chunk_solve<PO>(lf, lb, U, u, lane, Ny, chunk_column<1>(sh + 3 * ld, hs, ld, lane), maps);
+    maps.start(hf, U, u, lane, Ny);
+  }
+  // phase 3: R_c in r0, r1, r2 (through registers: the stencils read them)
+  {
+    cx<double> r[YP][3];
+#pragma unroll
+    for (int j0 = 0; j0 < YP; j0 += G) {
+      Weights<PO + 1> e1[G];
+      Weights<PO + 2> e2[G];
+#pragma unroll
+      for (int j = 0; j < G && j0 + j < YP; ++j) {
+        // opaque: else phase 1's weights wait in registers through the solve
+        const int y = opaque(min(lane + 64 * (j0 + j), Ny - 1));
+        e1[j] = Weights<PO + 1>(a.d1w, Ny, y);
+        e2[j] = Weights<PO + 2>(a.d2w, Ny, y);
+      }
+      if (j0 == 0) __syncthreads();  // p_P is there
+#pragma unroll
+      for (int j = 0; j < G && j0 + j < YP; ++j)
+        imm_r_at<PO>(a, e1[j], e2[j], r3, r0, ld, nc[j0 + j], kx, kz, k2, min(lane + 64 * (j0 + j), Ny - 1), r[j0 + j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    wave_sync();
+#pragma unroll
+    for (int j = 0; j < YP; ++j)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) r0[c * ld + min(lane + 64 * j, Ny - 1)] = r[j][c];
+  }
+  __syncthreads();
+  // phase 4: the arbitrary velocity in r0, r1, r2
+  if (solver) chunk_solve<PO>(hf, hb, U, u, lane, Ny, chunk_column<3>(sh, hs, ld, lane), maps);
+  // phase 5, its operands asked for before the barrier (the wavefront that
+  // does not solve has them by then)
+  double4 vq[YP];
+  cx<double> uj[YP][3];
+  double qw[YP];
+#pragma unroll
+  for (int j = 0; j < YP; ++j) {
+    const int y = opaque(min(lane + 64 * j, Ny - 1));
+    vq[j] = reinterpret_cast<const double4*>(a.vq)[(size_t)u * Ny + y];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) uj[j][c] = a.uj[c * comp + row + y];
+    qw[j] = a.qw[y];
+  }
+  __syncthreads();
+  if (!live) return;
   cx<double> al1, al2;
-  imm_alpha<PO>(a, m, sol + Ny, 1, al1, al2);
+  imm_alpha<PO>(a, m, r1, 1, al1, al2);
   double acc = 0.0;
-  for (int y = t; y < Ny; y += 32)
-    acc += a.qw[y] * imm_assemble_at(a, m, row, comp, kx, kz, sol, sol + Ny, sol + 2 * Ny, 1, al1, al2, y, live);
-  // the mode's 32 lanes: a fixed pairwise order
 #pragma unroll
-  for (int o = 16; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 32);
-  if (t == 0 && live && a.partials) a.partials[m] = acc;
+  for (int j = 0; j < YP; ++j) {
+    const int y = lane + 64 * j;
+    if (y < Ny) acc += qw[j] * imm_assemble_at(a, m, row, comp, kx, kz, vq[j], uj[j], r0, r1, r2, 1, al1, al2, y);
+  }
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+  if (lane == 0 && a.partials) a.partials[m] = acc;
 }
 
 // Phase 3 (flows/plane_couette.py:449-472): R_c for the three components
@@ -1917,8 +1941,10 @@ __global__ void __launch_bounds__(kImmT) k_imm_rc(ImmArgs a) {
   }
   __syncthreads();
   for (int y = threadIdx.x; y < Ny; y += blockDim.x) {
-    cx<double> r[3];
-    imm_r_at<PO>(a, pp, ur, row, comp, kx, kz, k2, y, r);
+    cx<double> nc[3], r[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) nc[c] = imm_n_at(a, c * comp + row + y);
+    imm_r_at<PO>(a, Weights<PO + 1>(a.d1w, Ny, y), Weights<PO + 2>(a.d2w, Ny, y), pp, ur, Ny, nc, kx, kz, k2, y, r);
 #pragma unroll
     for (int c = 0; c < 3; ++c) svec(a, V_R + c, m)[y * VS] = r[c];
   }
@@ -1940,8 +1966,11 @@ __global__ void __launch_bounds__(kImmT) k_imm_final(ImmArgs a) {
   cx<double> al1, al2;
   imm_alpha<PO>(a, m, va, VS, al1, al2);
   double acc = 0.0;
-  for (int y = threadIdx.x; y < Ny; y += blockDim.x)
-    acc += a.qw[y] * imm_assemble_at(a, m, row, comp, kx, kz, ua, va, wa, VS, al1, al2, y, true);
+  for (int y = threadIdx.x; y < Ny; y += blockDim.x) {
+    const double4 w = reinterpret_cast<const double4*>(a.vq)[(size_t)a.umode[m] * Ny + y];
+    const cx<double> uj[3] = {a.uj[row + y], a.uj[comp + row + y], a.uj[2 * comp + row + y]};
+    acc += a.qw[y] * imm_assemble_at(a, m, row, comp, kx, kz, w, uj, ua, va, wa, VS, al1, al2, y);
+  }
   const double s = block_sum(acc, red);
   if (threadIdx.x == 0 && a.partials) a.partials[m] = s;
 }
@@ -2082,11 +2111,9 @@ static int walls_imm(Ctx* c, const double* un, const double* uj, const double* n
   a.out = reinterpret_cast<cx<double>*>(out);
   a.corr = reinterpret_cast<cx<double>*>(corr);
   a.partials = c->partials;
-  a.d1w = t->d1w;
-  a.d2w = t->d2w;
+  a.d1w = t->d1t;
+  a.d2w = t->d2t;
   a.qw = t->qw;
-  a.d1j0 = t->d1j0;
-  a.d2j0 = t->d2j0;
   a.lk_ab = t->lk_ab;
   a.hk_ab = t->hk_ab;
   a.lk_piv = t->lk_piv;
@@ -2109,47 +2136,48 @@ static int walls_imm(Ctx* c, const double* un, const double* uj, const double* n
     ProfScope ps(c, KID_W_IMM, s);
     const size_t lds = (size_t)t->Ny * sizeof(cx<double>);
     const dim3 gm(t->M), gs((t->M + kSweepLanes - 1) / kSweepLanes, 1),
-        gs3((t->M + kSweepLanes - 1) / kSweepLanes, 3), gc((t->M + 1) / 2);
-    // chunked solves: per workgroup two modes' vectors and windows
-    const size_t lds_c1 = (size_t)2 * 1 * (t->Ny + 32) * sizeof(cx<double>);
-    const size_t lds_c3 = (size_t)2 * 3 * (t->Ny + 32) * sizeof(cx<double>);
-    if (4 * lds > 65536 || (!c->sweep_seq && lds_c3 > 65536))
+        gs3((t->M + kSweepLanes - 1) / kSweepLanes, 3), gc(t->items);
+    // chunked solves: per workgroup two modes' vectors
+    const size_t lds_c1 = (size_t)chunk_lds(t->Ny, t->p, 2) * sizeof(cx<double>);
+    const size_t lds_c3 = (size_t)chunk_lds(t->Ny, t->p, 6) * sizeof(cx<double>);
+    if (4 * lds > 65536 || (!c->sweep_seq && (size_t)2 * 3 * (t->Ny + 32) * sizeof(cx<double>) > 65536))
       return c->fail(DNSMI_EINVAL, "imm: ny too large for the per-mode LDS rows");
-    // the fused form reads u^n while other modes already store the new
-    // velocity: it needs them apart
-    if (c->imm_fused && !c->sweep_seq && out != un) {
-      const size_t lds_l = imm_lsolve_lds(t->Ny) * sizeof(cx<double>);
-      const size_t lds_h = imm_hsolve_lds(t->Ny) * sizeof(cx<double>);
-      if (lds_h > 65536) return c->fail(DNSMI_EINVAL, "imm: ny too large for the fused form's LDS rows");
-      switch (t->p) {
-#define IMMF(PO)                                                                                   \
-  case PO:                                                                                         \
-    hipLaunchKernelGGL((k_imm_lsolve<PO, chunk_slots(PO, 1)>), gc, dim3(64), lds_l, s, a, t->lk_fmap, \
-                       t->lk_bmap, t->sched, t->U);                                                \
-    hipLaunchKernelGGL((k_imm_hsolve<PO, chunk_slots(PO, 3)>), gc, dim3(64), lds_h, s, a, t->hk_fmap, \
-                       t->hk_bmap, t->sched, t->U);                                                \
+    if (c->imm_fused && !c->sweep_seq) {
+      if (t->Ny > kImmFusedNy) return c->fail(DNSMI_EINVAL, "imm: ny too large for the fused form");
+      const size_t lds_f = (size_t)chunk_lds(t->Ny, t->p, 2 * kImmRows) * sizeof(cx<double>);
+#define IMMF(PO, YP)                                                                                      \
+  hipLaunchKernelGGL((k_imm_fused<PO, YP>), gc, dim3(128), lds_f, s, a, t->lk_fmap, t->lk_bmap, \
+                     t->hk_fmap, t->hk_bmap, t->sched, t->U)
+#define IMMFP(PO)                       \
+  case PO:                              \
+    if (t->Ny <= 64) IMMF(PO, 1);       \
+    else if (t->Ny <= 128) IMMF(PO, 2); \
+    else if (t->Ny <= 256) IMMF(PO, 4); \
+    else IMMF(PO, 5);                   \
     break;
-        IMMF(2) IMMF(4) IMMF(6) IMMF(8)
-#undef IMMF
+      switch (t->p) {
+        IMMFP(2) IMMFP(4) IMMFP(6) IMMFP(8)
         default: return c->fail(DNSMI_EINVAL, "fd_order");
       }
+#undef IMMFP
+#undef IMMF
     } else
     switch (t->p) {
 #define IMM(PO)                                                                                   \
   case PO:                                                                                        \
-    hipLaunchKernelGGL(k_imm_fhat<PO>, gm, dim3(kImmT), 4 * lds, s, a);                           \
+    hipLaunchKernelGGL(k_imm_fhat<PO>, gm, dim3(kImmT), 3 * lds, s, a);                           \
     if (c->sweep_seq)                                                                             \
       hipLaunchKernelGGL(k_band_sweeps<PO>, gs, dim3(kSweepLanes), 0, s, a, t->lk_ab, t->lk_piv,   \
                          (int)V_F, (int)V_T, (int)V_P);                                           \
     else                                                                                          \
-      hipLaunchKernelGGL((k_band_chunks<PO, 1, chunk_slots(PO, 1)>), gc, dim3(64), lds_c1, s, a, t->lk_fmap,          \
+      hipLaunchKernelGGL((k_band_chunks<PO, 1>), gc, dim3(64), lds_c1, s, a, t->lk_fmap,          \
                          t->lk_bmap, t->sched, t->U, (int)V_F, (int)V_P);                         \
     hipLaunchKernelGGL(k_imm_rc<PO>, gm, dim3(kImmT), 4 * lds, s, a);                             \
     if (c->sweep_seq)                                                                             \
       hipLaunchKernelGGL(k_band_sweeps<PO>, gs3, dim3(kSweepLanes), 0, s, a, t->hk_ab, t->hk_piv, \
                          (int)V_R, (int)V_T, (int)V_R);                                           \
     else                                                                                          \
-      hipLaunchKernelGGL((k_band_chunks<PO, 3, chunk_slots(PO, 3)>), gc, dim3(64), lds_c3, s, a, t->hk_fmap,          \
+      hipLaunchKernelGGL((k_band_chunks<PO, 3>), gc, dim3(64), lds_c3, s, a, t->hk_fmap,          \
                          t->hk_bmap, t->sched, t->U, (int)V_R, (int)V_R);                         \
     hipLaunchKernelGGL(k_imm_final<PO>, gm, dim3(kImmT), 0, s, a);                                \
     break;
@@ -2310,7 +2338,7 @@ int walls_iterate_correction(Ctx* c, const double* state_prev, double* pred,
 // The set-up tables in the reference layouts (for tests), read back from the
 // device: which = 0 Lk_ab, 1 Hk_ab (mode, row, y), 2 v1, 3 q1 (mode, y),
 // 4 M_inv (mode, 2, 2), 5 ys; 6 Lk_piv, 7 Hk_piv (mode, y; ints written as
-// doubles); 8 .. 11 the packed chunk maps as stored (L_k forward, L_k back,
+// doubles); 8 .. 11 the chunk maps as stored (L_k forward, L_k back,
 // H_k forward, H_k back; empty without them); 12 the per-class homogeneous
 // solutions as stored ([class][y][4]); 13 the word counts of 8 .. 11 and
 // the number of k^2 classes.
@@ -2377,9 +2405,8 @@ int walls_table(Ctx* c, int which, double* out, long long n) {
     case 9:
     case 10:
     case 11: {
-      const int kl = t->p, B = kChunk, WF = B + kl, WB = B + 2 * kl, nC = (Ny + B - 1) / B;
-      const bool fwd = which == 8 || which == 10;
-      const size_t words = (size_t)nC * U * (fwd ? map_pre(WF, kl, WF) : map_pre(WB, 0, WB));
+      const bool back = which == 9 || which == 11;
+      const size_t words = (size_t)chunk_count(Ny, t->p, back) * U * map_words(t->p, back);
       const double* src = which == 8 ? t->lk_fmap : which == 9 ? t->lk_bmap : which == 10 ? t->hk_fmap : t->hk_bmap;
       if (!src) return want(0);
       if ((rc = want((long long)words))) return rc;
@@ -2389,10 +2416,9 @@ int walls_table(Ctx* c, int which, double* out, long long n) {
     case 13: {  // the words of tables 8 .. 11 (0 where absent), then the class count
       if ((rc = want(5))) return rc;
       out[4] = U;
-      const int kl = t->p, B = kChunk, WF = B + kl, WB = B + 2 * kl, nC = (Ny + B - 1) / B;
       const double* maps[4] = {t->lk_fmap, t->lk_bmap, t->hk_fmap, t->hk_bmap};
       for (int i = 0; i < 4; ++i)
-        out[i] = maps[i] ? (double)((size_t)nC * U * (i % 2 == 0 ? map_pre(WF, kl, WF) : map_pre(WB, 0, WB))) : 0.0;
+        out[i] = maps[i] ? (double)((size_t)chunk_count(Ny, t->p, i % 2 != 0) * U * map_words(t->p, i % 2 != 0)) : 0.0;
       return DNSMI_OK;
     }
     default: return c->fail(DNSMI_EINVAL, "unknown table");

@@ -77,8 +77,8 @@ typedef struct dnsmi_config {
   int variants;            /* bit mask when tile_cols != 0: 1 sequential
                               y-inverse, 2 sequential z-inverse, 4 split x pass,
                               8 sequential band sweeps (walls; else chunk maps),
-                              16 the chunk maps' fused two-launch influence-
-                              matrix step (walls, without 8), 32 non-temporal
+                              16 the chunk maps' one-launch influence-matrix
+                              step (walls, without 8), 32 non-temporal
                               stores of the z-inverse output (periodic), 64
                               64-row workgroups of the FD curl (walls) */
   int plain_mixed;         /* DNSMI_MIXED only: 0 (default) evaluates every
@@ -169,7 +169,7 @@ int dnsmi_variants(const dnsmi_ctx* ctx, int* tile_cols, int* variants);
  * keeps these as module attributes, flows/plane_couette.py:139-219):
  * which = 0 Lk_ab (Nkz,Nkx,3p+1,Ny), 1 Hk_ab, 2 v1 (Nkz,Nkx,Ny), 3 q1,
  * 4 M_inv (Nkz,Nkx,2,2), 5 y grid (Ny), 6 Lk_piv, 7 Hk_piv (0-based pivots
- * as doubles); as stored on the device: 8 .. 11 the packed chunk maps of the
+ * as doubles); as stored on the device: 8 .. 11 the chunk maps of the
  * L_k forward, L_k back, H_k forward and H_k back solves, 12 the per-class
  * homogeneous solutions ([class][y][v1, v2, q1, q2]), 13 the word counts of
  * tables 8 .. 11 (0 where a table is absent) and the number of k^2 classes
