@@ -1007,17 +1007,191 @@ __global__ void __launch_bounds__(TC * ColPlan<P>::threads) k_z_forward_b(const 
 
 
 // ------------------------------------------------------------------ K5
+// The epilogue's operands at one mode: what the mode of the pass combines
+// with the projected N, for the three components.
+template <int MODE>
+struct YOps {
+  cx<double> a[3];  // state, N_prev or B
+  cx<double> p[3];  // the iterate
+  cx<double> r[3];  // N(u_ref) of an increment
+  __device__ __forceinline__ void load(const StepArgs& g, size_t pos, size_t comp) {
+    constexpr bool predict = MODE == MODE_PREDICT || MODE == MODE_PREDICT_CARRY;
+    constexpr bool correct = MODE == MODE_CORRECT || MODE == MODE_CORRECT_CARRY;
+    const double* pa = predict ? g.state : (MODE == MODE_CORRECT_CARRY && g.nref ? g.nref : g.rhs_prev);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const size_t idx = c * comp + pos;
+      if constexpr (predict || correct) a[c] = reinterpret_cast<const cx<double>*>(pa)[idx];
+      if constexpr (correct) p[c] = reinterpret_cast<const cx<double>*>(g.pred)[idx];
+      if constexpr (MODE == MODE_RHS || MODE == MODE_PREDICT || MODE == MODE_CORRECT)
+        if (g.nref) r[c] = reinterpret_cast<const cx<double>*>(g.nref)[idx];
+    }
+  }
+};
+
+// One mode: the projection of N and the pass's update of the three
+// components.  Returns the mode's share of the norm.
+template <int MODE>
+__device__ __forceinline__ double y_epilogue(const StepArgs& args, const YOps<MODE>& cur, cx<double> n0,
+                                             cx<double> n1, cx<double> n2, double kxv, double kyv, double kzv,
+                                             double km, bool mean, size_t pos, size_t comp) {
+  double acc = 0.0;
+  const double lapl = -((kxv * kxv + kyv * kyv) + kzv * kzv);
+  const double il = lapl < 0 ? 1.0 / lapl : 0.0;
+  // div = i kx N0 + i ky N1 + i kz N2 ; p = inv_lapl * div
+  const cx<double> dv = {((-kxv * n0.y) + (-kyv * n1.y)) + (-kzv * n2.y),
+                         ((kxv * n0.x) + (kyv * n1.x)) + (kzv * n2.x)};
+  const cx<double> pr = {il * dv.x, il * dv.y};
+  const double kk[3] = {kxv, kyv, kzv};
+  const cx<double> nn[3] = {n0, n1, n2};
+  const double ldt1 = mean ? 0.0 : 1.0 / args.dt + (1.0 - args.c) * lapl / args.re;
+  const double ildt2 = mean ? 0.0 : 1.0 / (1.0 / args.dt - args.c * lapl / args.re);
+  cx<double>* pd = reinterpret_cast<cx<double>*>(args.pred);
+  cx<double>* rout = reinterpret_cast<cx<double>*>(args.rhs_out);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    // rhs = N - i k p (increments: N(u_ref) + P[dN])
+    cx<double> rh = {nn[c].x + kk[c] * pr.y, nn[c].y - kk[c] * pr.x};
+    const size_t idx = c * comp + pos;
+    if constexpr (MODE == MODE_CORRECT_CARRY) {
+      // u <- B + c ildt_2 N(u); increments: (B + c ildt_2 N(u_ref)) + c ildt_2 P[dN]
+      const cx<double> base = cur.a[c], p0 = cur.p[c];
+      const double ci = args.c * ildt2;
+      const cx<double> un = {base.x + ci * rh.x, base.y + ci * rh.y};
+      const cx<double> d = {un.x - p0.x, un.y - p0.y};
+      pd[idx] = un;
+      if (args.nref_out) reinterpret_cast<cx<double>*>(args.nref_out)[idx] = un;
+      acc += km * (d.x * d.x) + km * (d.y * d.y);
+      continue;
+    }
+    if constexpr (MODE == MODE_PREDICT_CARRY) {
+      const cx<double> u = cur.a[c];
+      pd[idx] = {(u.x * ldt1 + rh.x) * ildt2, (u.y * ldt1 + rh.y) * ildt2};
+      const double cm = 1.0 - args.c;
+      rout[idx] = {(u.x * ldt1 + cm * rh.x) * ildt2, (u.y * ldt1 + cm * rh.y) * ildt2};
+      continue;
+    }
+    if (args.nref) rh = {cur.r[c].x + rh.x, cur.r[c].y + rh.y};
+    if (args.nref_out) reinterpret_cast<cx<double>*>(args.nref_out)[idx] = rh;
+    if constexpr (MODE == MODE_PREDICT) {
+      const cx<double> u = cur.a[c];
+      pd[idx] = {(u.x * ldt1 + rh.x) * ildt2, (u.y * ldt1 + rh.y) * ildt2};
+    } else if constexpr (MODE == MODE_CORRECT) {
+      const cx<double> np = cur.a[c], p0 = cur.p[c];
+      const cx<double> d = {args.c * (rh.x - np.x) * ildt2, args.c * (rh.y - np.y) * ildt2};
+      pd[idx] = {p0.x + d.x, p0.y + d.y};
+      acc += km * (d.x * d.x) + km * (d.y * d.y);
+    }
+    rout[idx] = rh;
+  }
+  return acc;
+}
+
+// A third of the workgroup per component: the three transforms run side by
+// side, meet in LDS, and the projection and epilogue then go over the modes
+// with all threads, three components to a thread, the next mode's operands
+// loaded before this one's results are stored.
+//
+// The pass has one workgroup per column tile (62 at 32^3, 508 at 128^3), so
+// below the largest grids it is bound by one workgroup's chain of memory round
+// trips: three transforms and 36 epilogue loads one behind the other in the
+// serial form (below), one transform and at most three modes here.  A launch,
+// serial and side by side: 32^3 FP64 11.1 and 5.7 us, 64^3 FP64 15.8 and 7.9,
+// 96 x 64 x 48 FP32 23.5 and 11.0, sixteen 48^3 FP32 54.5 and 40.9; 128^3 FP32
+// moves its 224 MB at memory speed either way (55.0 and 56.8 us).
 template <typename T, int P, int TC, int MODE, bool PADY>
 __device__ __forceinline__ void y_forward_body(const cx<T>* __restrict__ w4, const cx<T>* __restrict__ tw,
                 const double* __restrict__ kx_tab, const double* __restrict__ ky_tab,
                 const double* __restrict__ kz_tab, int ny, int Nz1, int Nx1, StepArgs args) {
   if (args.act && *args.act == 0) return;
   constexpr int N1 = ColPlan<P>::N1, N2 = ColPlan<P>::N2;
-  __shared__ cx<T> lds[TC * P];
+  constexpr int NM = PADY ? 2 * P / 3 : P;    // ny
+  constexpr int G = 3 * N2;                   // threads of one column
+  constexpr int IT = (NM - 1 + G - 1) / G;    // modes of one thread
+  __shared__ cx<T> lds[3 * TC * P];
   __shared__ cx<T> tws[P];
+  __shared__ double red[16];
   for (int i = threadIdx.x; i < P; i += blockDim.x) tws[i] = tw[i];
   __syncthreads();
+  const int tid = threadIdx.x, col = tid % TC, g = tid / TC;
+  const int tc = g / N2, j = g - tc * N2;
+  const int ntile = (Nx1 + TC - 1) / TC;
+  const int kz = blockIdx.x / ntile;
+  const int kx = (blockIdx.x - kz * ntile) * TC + col;
+  const bool ok = kx < Nx1;
+  const size_t plane = (size_t)Nz1 * Nx1;
+  const size_t in_f = (size_t)P * plane;
+  const size_t off = (size_t)kz * Nx1 + kx;
+  const size_t comp = (size_t)(ny - 1) * plane;
+  const T inv = static_cast<T>(1.0 / P);
+  cx<T>* lc = lds + tc * (TC * P);
+  {
+    cx<T> x[N1];
+#pragma unroll
+    for (int a = 0; a < N1; ++a)
+      x[a] = ok ? w4[tc * in_f + (size_t)(N2 * a + j) * plane + off] : cx<T>{0, 0};
+    step_a_store<P, N1, N2, -1, TC>(x, j, col, lc, tws);
+  }
+  YOps<MODE> cur;
+  if (ok && g < NM - 1) cur.load(args, (size_t)g * plane + off, comp);
+  __syncthreads();
+  {
+    cx<T> R[N2];
+    if (j < N1) step_b_load<P, N1, N2, -1, TC>(R, j, col, lc);
+    __syncthreads();
+    if (j < N1) {
+#pragma unroll
+      for (int k2 = 0; k2 < N2; ++k2)
+        if (!PadN<P, NM>::zero(N1 * k2, N1 * k2 + N1 - 1)) lc[(j + N1 * k2) * TC + col] = cscale(R[k2], inv);
+    }
+  }
+  __syncthreads();
+
+  double acc = 0.0;
+  const double kxv = ok ? kx_tab[kx] : 0.0, kzv = kz_tab[kz];
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int s = g + it * G;
+    YOps<MODE> nxt;
+    if (it + 1 < IT && ok && s + G < NM - 1) nxt.load(args, (size_t)(s + G) * plane + off, comp);
+    if (ok && s < NM - 1) {
+      const int m = s < NM / 2 ? s : s + (P - NM + 1);
+      const cx<T>* l = lds + m * TC + col;
+      acc += y_epilogue<MODE>(args, cur, {l[0].x, l[0].y}, {l[TC * P].x, l[TC * P].y},
+                              {l[2 * TC * P].x, l[2 * TC * P].y}, kxv, ky_tab[s], kzv, kx == 0 ? 1.0 : 2.0,
+                              s == 0 && kz == 0 && kx == 0, (size_t)s * plane + off, comp);
+    }
+    cur = nxt;
+  }
+  if (MODE == MODE_CORRECT || MODE == MODE_CORRECT_CARRY) {
+    const double s = block_sum(acc, red);
+    if (threadIdx.x == 0) args.partials[blockIdx.x] = s;
+  }
+}
+template <typename T, int P, int TC, int MODE, bool PADY>
+__global__ void __launch_bounds__(3 * TC * ColPlan<P>::threads) k_y_forward(YFwdArgs a) {
+  y_forward_body<T, P, TC, MODE, PADY>(static_cast<const cx<T>*>(a.w4), static_cast<const cx<T>*>(a.tw), a.kx, a.ky, a.kz, a.ny, a.Nz1, a.Nx1, a.s);
+}
+template <typename T, int P, int TC, int MODE, bool PADY>
+__global__ void __launch_bounds__(3 * TC * ColPlan<P>::threads) k_y_forward_b(const YFwdArgs* __restrict__ t) {
+  const YFwdArgs a = t[blockIdx.z];
+  y_forward_body<T, P, TC, MODE, PADY>(static_cast<const cx<T>*>(a.w4), static_cast<const cx<T>*>(a.tw), a.kx, a.ky, a.kz, a.ny, a.Nz1, a.Nx1, a.s);
+}
+
+
+// The components one behind the other in one tile's LDS, the results in
+// registers.
+template <typename T, int P, int TC, int MODE, bool PADY>
+__device__ __forceinline__ void y_forward_serial_body(const cx<T>* __restrict__ w4, const cx<T>* __restrict__ tw,
+                const double* __restrict__ kx_tab, const double* __restrict__ ky_tab,
+                const double* __restrict__ kz_tab, int ny, int Nz1, int Nx1, StepArgs args) {
+  if (args.act && *args.act == 0) return;
+  constexpr int N1 = ColPlan<P>::N1, N2 = ColPlan<P>::N2;
+  __shared__ cx<T> lds[TC * P];
+  __shared__ cx<T> tws[P];
   __shared__ double red[16];
+  for (int i = threadIdx.x; i < P; i += blockDim.x) tws[i] = tw[i];
+  __syncthreads();
   const int tid = threadIdx.x, col = tid % TC, j = tid / TC;
   const int ntile = (Nx1 + TC - 1) / TC;
   const int kz = blockIdx.x / ntile;
@@ -1050,77 +1224,15 @@ __device__ __forceinline__ void y_forward_body(const cx<T>* __restrict__ w4, con
   double acc = 0.0;
   if (j < N1 && ok) {
     const double kxv = kx_tab[kx], kzv = kz_tab[kz];
-    const double km = kx == 0 ? 1.0 : 2.0;
 #pragma unroll
     for (int k2 = 0; k2 < N2; ++k2) {
       const int s = PadN<P, PADY ? 2 * P / 3 : P>::stored_in(N1 * k2, N1, j);
       if (s < 0) continue;
-      const double kyv = ky_tab[s];
-      const double lapl = -((kxv * kxv + kyv * kyv) + kzv * kzv);
-      const double il = lapl < 0 ? 1.0 / lapl : 0.0;
-      const cx<double> n0 = {R[0][k2].x, R[0][k2].y};
-      const cx<double> n1 = {R[1][k2].x, R[1][k2].y};
-      const cx<double> n2 = {R[2][k2].x, R[2][k2].y};
-      // div = i kx N0 + i ky N1 + i kz N2 ; p = inv_lapl * div
-      const cx<double> dv = {((-kxv * n0.y) + (-kyv * n1.y)) + (-kzv * n2.y),
-                             ((kxv * n0.x) + (kyv * n1.x)) + (kzv * n2.x)};
-      const cx<double> pr = {il * dv.x, il * dv.y};
-      const double kk[3] = {kxv, kyv, kzv};
-      const cx<double> nn[3] = {n0, n1, n2};
-      const bool mean = (s == 0 && kz == 0 && kx == 0);
-      const double ldt1 = mean ? 0.0 : 1.0 / args.dt + (1.0 - args.c) * lapl / args.re;
-      const double ildt2 = mean ? 0.0 : 1.0 / (1.0 / args.dt - args.c * lapl / args.re);
-      const size_t pos = (size_t)s * plane + off;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        // rhs = N - i k p (increments: N(u_ref) + P[dN])
-        cx<double> rh = {nn[c].x + kk[c] * pr.y, nn[c].y - kk[c] * pr.x};
-        const size_t idx = c * comp + pos;
-        if constexpr (MODE == MODE_CORRECT_CARRY) {
-          // u <- B + c ildt_2 N(u); increments: (B + c ildt_2 N(u_ref)) + c ildt_2 P[dN]
-          const cx<double> base = reinterpret_cast<const cx<double>*>(args.nref ? args.nref : args.rhs_prev)[idx];
-          const double ci = args.c * ildt2;
-          const cx<double> un = {base.x + ci * rh.x, base.y + ci * rh.y};
-          cx<double>* pd = reinterpret_cast<cx<double>*>(args.pred);
-          const cx<double> p0 = pd[idx];
-          const cx<double> d = {un.x - p0.x, un.y - p0.y};
-          pd[idx] = un;
-          if (args.nref_out) reinterpret_cast<cx<double>*>(args.nref_out)[idx] = un;
-          acc += km * (d.x * d.x) + km * (d.y * d.y);
-          continue;
-        }
-        if constexpr (MODE == MODE_PREDICT_CARRY) {
-          const cx<double> u = reinterpret_cast<const cx<double>*>(args.state)[idx];
-          cx<double>* pd = reinterpret_cast<cx<double>*>(args.pred);
-          cx<double>* rout = reinterpret_cast<cx<double>*>(args.rhs_out);
-          pd[idx] = {(u.x * ldt1 + rh.x) * ildt2, (u.y * ldt1 + rh.y) * ildt2};
-          const double cm = 1.0 - args.c;
-          rout[idx] = {(u.x * ldt1 + cm * rh.x) * ildt2, (u.y * ldt1 + cm * rh.y) * ildt2};
-          continue;
-        }
-        if (args.nref) {
-          const cx<double> r0 = reinterpret_cast<const cx<double>*>(args.nref)[idx];
-          rh = {r0.x + rh.x, r0.y + rh.y};
-        }
-        if (args.nref_out) reinterpret_cast<cx<double>*>(args.nref_out)[idx] = rh;
-        cx<double>* rout = reinterpret_cast<cx<double>*>(args.rhs_out);
-        if (MODE == MODE_RHS) {
-          rout[idx] = rh;
-        } else if (MODE == MODE_PREDICT) {
-          const cx<double> u = reinterpret_cast<const cx<double>*>(args.state)[idx];
-          cx<double>* pd = reinterpret_cast<cx<double>*>(args.pred);
-          pd[idx] = {(u.x * ldt1 + rh.x) * ildt2, (u.y * ldt1 + rh.y) * ildt2};
-          rout[idx] = rh;
-        } else {
-          const cx<double> np = reinterpret_cast<const cx<double>*>(args.rhs_prev)[idx];
-          cx<double>* pd = reinterpret_cast<cx<double>*>(args.pred);
-          const cx<double> d = {args.c * (rh.x - np.x) * ildt2, args.c * (rh.y - np.y) * ildt2};
-          const cx<double> p0 = pd[idx];
-          pd[idx] = {p0.x + d.x, p0.y + d.y};
-          rout[idx] = rh;
-          acc += km * (d.x * d.x) + km * (d.y * d.y);
-        }
-      }
+      YOps<MODE> ops;
+      ops.load(args, (size_t)s * plane + off, comp);
+      acc += y_epilogue<MODE>(args, ops, {R[0][k2].x, R[0][k2].y}, {R[1][k2].x, R[1][k2].y},
+                              {R[2][k2].x, R[2][k2].y}, kxv, ky_tab[s], kzv, kx == 0 ? 1.0 : 2.0,
+                              s == 0 && kz == 0 && kx == 0, (size_t)s * plane + off, comp);
     }
   }
   if (MODE == MODE_CORRECT || MODE == MODE_CORRECT_CARRY) {
@@ -1129,13 +1241,13 @@ __device__ __forceinline__ void y_forward_body(const cx<T>* __restrict__ w4, con
   }
 }
 template <typename T, int P, int TC, int MODE, bool PADY>
-__global__ void __launch_bounds__(TC * ColPlan<P>::threads) k_y_forward(YFwdArgs a) {
-  y_forward_body<T, P, TC, MODE, PADY>(static_cast<const cx<T>*>(a.w4), static_cast<const cx<T>*>(a.tw), a.kx, a.ky, a.kz, a.ny, a.Nz1, a.Nx1, a.s);
+__global__ void __launch_bounds__(TC * ColPlan<P>::threads) k_y_forward_serial(YFwdArgs a) {
+  y_forward_serial_body<T, P, TC, MODE, PADY>(static_cast<const cx<T>*>(a.w4), static_cast<const cx<T>*>(a.tw), a.kx, a.ky, a.kz, a.ny, a.Nz1, a.Nx1, a.s);
 }
 template <typename T, int P, int TC, int MODE, bool PADY>
-__global__ void __launch_bounds__(TC * ColPlan<P>::threads) k_y_forward_b(const YFwdArgs* __restrict__ t) {
+__global__ void __launch_bounds__(TC * ColPlan<P>::threads) k_y_forward_serial_b(const YFwdArgs* __restrict__ t) {
   const YFwdArgs a = t[blockIdx.z];
-  y_forward_body<T, P, TC, MODE, PADY>(static_cast<const cx<T>*>(a.w4), static_cast<const cx<T>*>(a.tw), a.kx, a.ky, a.kz, a.ny, a.Nz1, a.Nx1, a.s);
+  y_forward_serial_body<T, P, TC, MODE, PADY>(static_cast<const cx<T>*>(a.w4), static_cast<const cx<T>*>(a.tw), a.kx, a.ky, a.kz, a.ny, a.Nz1, a.Nx1, a.s);
 }
 
 
@@ -1326,6 +1438,7 @@ static void with_tc(const Ctx* c, F&& f) {
     f(std::integral_constant<int, kTC>{});
 }
 constexpr int kRows = 16;  // rows per workgroup of the x pass
+constexpr int kCUs = 256;   // compute units of the chip
 
 template <typename T, int P, int EM, int TC>
 static void launch_y_inverse_p(Ctx* c, dim3 grid, const cx<double>* u, cx<T>* w1, const cx<T>* tw,
@@ -1504,6 +1617,24 @@ static int launch_z_forward(Ctx* c, hipStream_t s) {
   return launch_z_forward_buf<T>(c, b.A, b.B, c->Py, KID_Z_FORWARD, s);
 }
 
+template <typename T, int P, int TC, int MODE, bool PADY>
+static void launch_y_forward_p(Ctx* c, int nb, const YFwdArgs& a, hipStream_t s) {
+  // Three components of 16 columns that take more than half a CU's LDS leave
+  // one workgroup to it: with more workgroups than CUs nothing overlaps one's
+  // transforms with another's loads, and the serial form is the faster one.
+  // FP64 step at 128^3 (508 workgroups): 786 us serial, 789 us side by side;
+  // 64 x 128^2 (254): 449 us serial, 411 us side by side.
+  if constexpr (3 * TC * P * sizeof(cx<T>) > 80 * 1024) {
+    if (nb > kCUs) {
+      launch(c, &k_y_forward_serial<T, P, TC, MODE, PADY>, &k_y_forward_serial_b<T, P, TC, MODE, PADY>, dim3(nb),
+             dim3(TC * ColPlan<P>::threads), s, a);
+      return;
+    }
+  }
+  launch(c, &k_y_forward<T, P, TC, MODE, PADY>, &k_y_forward_b<T, P, TC, MODE, PADY>, dim3(nb),
+         dim3(3 * TC * ColPlan<P>::threads), s, a);
+}
+
 template <typename T, int MODE>
 static int launch_y_forward(Ctx* c, const StepArgs& a, hipStream_t s, int* nblocks) {
   Bufs<T> b = bufs_of<T>(c);
@@ -1513,18 +1644,16 @@ static int launch_y_forward(Ctx* c, const StepArgs& a, hipStream_t s, int* nbloc
   if ((MODE == MODE_CORRECT || MODE == MODE_CORRECT_CARRY) && nb > c->max_partials)
     return c->fail(DNSMI_EINVAL, "y_forward: too many blocks");
   ProfScope ps(c, KID_Y_FORWARD, s);
+  const YFwdArgs ya{b.B, b.twy, c->kx, c->ky, c->kz, c->ny, c->Nz1, c->Nx1, a};
   switch (c->Py) {
 #define X(P)                                                                                   \
   case P:                                                                                      \
     with_tc(c, [&](auto tcv) {                                                                 \
       constexpr int TC = decltype(tcv)::value;                                                 \
-      const YFwdArgs ya{b.B, b.twy, c->kx, c->ky, c->kz, c->ny, c->Nz1, c->Nx1, a};           \
       if (c->Py != c->ny)                                                                      \
-        launch(c, &k_y_forward<T, P, TC, MODE, true>, &k_y_forward_b<T, P, TC, MODE, true>,    \
-               dim3(nb), dim3(TC * ColPlan<P>::threads), s, ya);                               \
+        launch_y_forward_p<T, P, TC, MODE, true>(c, nb, ya, s);                                \
       else                                                                                     \
-        launch(c, &k_y_forward<T, P, TC, MODE, false>, &k_y_forward_b<T, P, TC, MODE, false>,  \
-               dim3(nb), dim3(TC * ColPlan<P>::threads), s, ya);                               \
+        launch_y_forward_p<T, P, TC, MODE, false>(c, nb, ya, s);                               \
     });                                                                                        \
     break;
     DNSMI_FOR_EACH_P(X)
