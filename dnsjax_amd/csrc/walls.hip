@@ -1773,8 +1773,8 @@ __global__ void __launch_bounds__(64, 2)
 // values, bit for bit); eight work vectors' round trips through memory and
 // four launches go.
 //
-// Traffic: 15 vector components, and a class's maps for every two modes (860
-// bytes per point at p = 6: more than the fields).  The maps' way from the
+// Traffic: 15 vector components, and a class's maps for every two modes (1140
+// bytes per point at p = 6, where the fields of both are 480).  The maps' way from the
 // caches is the bound, not the products, which would take 20 us per item at
 // Ny = 256, p = 6; four items per CU (36 KB of LDS, 256 registers) put one
 // solving wavefront on each SIMD (the first wavefronts of a CU's workgroups
