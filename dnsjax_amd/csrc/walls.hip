@@ -215,28 +215,55 @@ static void band_solve(const Band& B, std::vector<double>& b) {
 // 16 rows, or of 32 where a back window's reach leaves 16 too little (p >= 6).
 // B is a multiple of four rows, so that the rows a window keeps move by whole
 // registers of the matrix cores' operands (chunk_chain).
-__host__ __device__ constexpr int chunk_tiles(int p, bool back) { return back && p >= 6 ? 2 : 1; }
-__host__ __device__ constexpr int chunk_rows(int p, bool back) {
-  return 16 * chunk_tiles(p, back) - ((back ? 2 * p : p) + 3) / 4 * 4;
+//
+// mx, a mixed context: 16 rows, in windows of up to 32.  There the iterate is
+// rounded to FP32 at the start of every evaluation, where a change in its last
+// bit can send an element to the other neighbour: 1e-7 of the RMS in an
+// element of the nonlinear term, 1e-10 of the whole.  So the mixed form keeps
+// one order of operations to the bit: chunks of 16 rows, each of a map's sums
+// over the window's rows in ascending order (v_mfma_f64_16x16x4_f64 is four
+// fused multiply-adds in ascending k), and the right-hand sides' terms one by
+// one (imm_fhat_mx_at, imm_r_at).  Its maps take 80 words per row of the
+// column where the FP64 contexts' take 53 (p = 4; p = 6: 96 and 70), and one step
+// of 128 x 256 x 128, p = 6, 336 us where theirs takes 296.
+__host__ __device__ constexpr int chunk_tiles(int p, bool back, bool mx) { return mx || (back && p >= 6) ? 2 : 1; }
+__host__ __device__ constexpr int chunk_keep(int p, bool back) { return back ? 2 * p : p; }
+__host__ __device__ constexpr int chunk_rows(int p, bool back, bool mx) {
+  return mx ? 16 : 16 * chunk_tiles(p, back, mx) - (chunk_keep(p, back) + 3) / 4 * 4;
 }
-__host__ __device__ constexpr int chunk_window(int p, bool back) { return chunk_rows(p, back) + (back ? 2 * p : p); }
-__host__ __device__ constexpr int chunk_count(int n, int p, bool back) {
-  return (n + chunk_rows(p, back) - 1) / chunk_rows(p, back);
+__host__ __device__ constexpr int chunk_window(int p, bool back, bool mx) {
+  return chunk_rows(p, back, mx) + chunk_keep(p, back);
+}
+// rows that a window's registers hold: the window up to a multiple of four
+__host__ __device__ constexpr int chunk_span(int p, bool back, bool mx) {
+  return (chunk_window(p, back, mx) + 3) / 4 * 4;
+}
+__host__ __device__ constexpr int chunk_count(int n, int p, bool back, bool mx) {
+  return (n + chunk_rows(p, back, mx) - 1) / chunk_rows(p, back, mx);
 }
 // A map's words, in the order the products take them (map of chunk c, class
 // u at (c U + u) words): operand e of lane (g = lane / 16, r = lane % 16) at
 // map_word(e, lane), two operands side by side, so that a wavefront's load
 // is 1 KB of consecutive words.  One tile: e = k / 4, entry (t = r, k = 4 e +
-// g).  Two: e < 8 rows 16 + r, e = 8 .. 11 rows r, of which k >= 16 is zero by
-// construction (a back map is lower triangular) and left out.
-__host__ __device__ constexpr int map_operands(int p, bool back) { return chunk_tiles(p, back) == 1 ? 4 : 12; }
-__host__ __device__ constexpr int map_words(int p, bool back) { return 64 * map_operands(p, back); }
+// g).  Two: first the operands of rows 16 + r (high_operands), then those of
+// rows r (low_operands), of which a back map's k >= 16 are zero by construction
+// (it is lower triangular) and left out; an odd count is filled up with zeros.
+__host__ __device__ constexpr int high_operands(int p, bool back, bool mx) {
+  return chunk_tiles(p, back, mx) == 1 ? 0 : chunk_span(p, back, mx) / 4;
+}
+__host__ __device__ constexpr int low_operands(int p, bool back, bool mx) {
+  return back || !mx ? 4 : chunk_span(p, back, mx) / 4;
+}
+__host__ __device__ constexpr int map_operands(int p, bool back, bool mx) {
+  return (high_operands(p, back, mx) + low_operands(p, back, mx) + 1) / 2 * 2;
+}
+__host__ __device__ constexpr int map_words(int p, bool back, bool mx) { return 64 * map_operands(p, back, mx); }
 __host__ __device__ constexpr int map_word(int e, int lane) { return ((e >> 1) * 64 + lane) * 2 + (e & 1); }
-// entry (t, k) of word i, and back: -1 where it is left out
-__host__ __device__ inline void map_entry(int i, bool two, int& t, int& k) {
+// entry (t, k) of word i (k past the window where it is filled up)
+__host__ __device__ inline void map_entry(int i, int high, int& t, int& k) {
   const int e = (i >> 7) * 2 + (i & 1), lane = (i & 127) >> 1;
-  t = (lane & 15) + (two && e < 8 ? 16 : 0);
-  k = 4 * (two && e >= 8 ? e - 8 : e) + (lane >> 4);
+  t = (lane & 15) + (e < high ? 16 : 0);
+  k = 4 * (e < high ? e : e - high) + (lane >> 4);
 }
 
 // Chunk maps of one band solve (the operation order of band_solve): forward
@@ -249,25 +276,24 @@ __host__ __device__ inline void map_entry(int i, bool two, int& t, int& k) {
 // the pivot row.  Returns false if an entry left out is not zero (it cannot
 // be, by the argument above; the check keeps the layout honest).
 template <typename Raw, typename Piv>
-static bool chunk_maps(int n, int p, int u, int U, Raw raw, Piv piv, double* F, double* G) {
+static bool chunk_maps(int n, int p, bool mx, int u, int U, Raw raw, Piv piv, double* F, double* G) {
   const int kl = p, kuu = 2 * p;
   bool ok = true;
   std::vector<double> X;
   auto write = [&](bool back, int c, double* out) {
-    const int W = chunk_window(p, back), words = map_words(p, back);
-    const bool two = chunk_tiles(p, back) == 2;
+    const int W = chunk_window(p, back, mx), words = map_words(p, back, mx), high = high_operands(p, back, mx);
+    const int klow = 4 * low_operands(p, back, mx);  // columns that rows 0 .. 15 keep
     double* m = out + ((size_t)c * U + u) * words;
     for (int i = 0; i < words; ++i) {
       int t, k;
-      map_entry(i, two, t, k);
+      map_entry(i, high, t, k);
       m[i] = t < W && k < W ? X[(size_t)t * W + k] : 0.0;
     }
-    if (two)
-      for (int t = 0; t < 16; ++t)
-        for (int k = 16; k < W; ++k) ok = ok && X[(size_t)t * W + k] == 0.0;
+    for (int t = 0; t < 16 && t < W; ++t)
+      for (int k = klow; k < W; ++k) ok = ok && X[(size_t)t * W + k] == 0.0;
   };
-  for (int c = 0; c < chunk_count(n, p, false); ++c) {
-    const int B = chunk_rows(p, false), W = chunk_window(p, false), j0 = c * B;
+  for (int c = 0; c < chunk_count(n, p, false, mx); ++c) {
+    const int B = chunk_rows(p, false, mx), W = chunk_window(p, false, mx), j0 = c * B;
     X.assign((size_t)W * W, 0.0);
     for (int t = 0; t < W; ++t) X[(size_t)t * W + t] = 1.0;
     for (int j = j0; j < std::min(j0 + B, n - 1); ++j) {
@@ -281,8 +307,8 @@ static bool chunk_maps(int n, int p, int u, int U, Raw raw, Piv piv, double* F, 
     }
     write(false, c, F);
   }
-  for (int c = 0; c < chunk_count(n, p, true); ++c) {
-    const int B = chunk_rows(p, true), W = chunk_window(p, true), T = n - 1 - c * B;
+  for (int c = 0; c < chunk_count(n, p, true, mx); ++c) {
+    const int B = chunk_rows(p, true, mx), W = chunk_window(p, true, mx), T = n - 1 - c * B;
     X.assign((size_t)W * W, 0.0);
     for (int t = 0; t < W; ++t) X[(size_t)t * W + t] = 1.0;
     for (int j = T; j > T - B && j >= 0; --j) {
@@ -368,6 +394,7 @@ static int walls_autotune(Ctx* c);
 // factored and used.
 struct GpuSetup {
   int n, kl, ku, rows, U, W1, W2;  // W1, W2: widths of the D1 and D2 stencils
+  int mx;                          // chunk maps of a mixed context
   const double* d1w;
   const int* d1j0;
   const double* d2w;
@@ -578,10 +605,11 @@ __global__ void __launch_bounds__(64) k_setup_maps(GpuSetup g, double* lf, doubl
   const int c = blockIdx.x, u = blockIdx.y, which = blockIdx.z >> 1;
   const bool back = blockIdx.z & 1;
   const int lane = threadIdx.x, n = g.n, kl = g.kl, kuu = g.kl + g.ku;
-  if (c >= chunk_count(n, kl, back)) return;
+  const bool mx = g.mx;
+  if (c >= chunk_count(n, kl, back, mx)) return;
   const double* ab = g.band + (size_t)(which * g.U + u) * g.rows * n;
   const int* pv = g.piv + (size_t)(which * g.U + u) * n;
-  const int B = chunk_rows(kl, back), W = chunk_window(kl, back);
+  const int B = chunk_rows(kl, back, mx), W = chunk_window(kl, back, mx);
   for (int e = lane; e < W * W; e += 64) X[e] = (e / W == e % W) ? 1.0 : 0.0;
   __syncthreads();
   const int j0 = c * B;
@@ -623,17 +651,17 @@ __global__ void __launch_bounds__(64) k_setup_maps(GpuSetup g, double* lf, doubl
       __syncthreads();
     }
   }
-  const int words = map_words(kl, back);
-  const bool two = chunk_tiles(kl, back) == 2;
+  const int words = map_words(kl, back, mx), high = high_operands(kl, back, mx);
+  const int klow = 4 * low_operands(kl, back, mx);
   double* F = (which == 0 ? (back ? lb : lf) : (back ? hb : hf)) + ((size_t)c * g.U + u) * words;
   for (int i = lane; i < words; i += 64) {
     int t, k;
-    map_entry(i, two, t, k);
+    map_entry(i, high, t, k);
     F[i] = t < W && k < W ? X[t * W + k] : 0.0;
   }
   bool bad = false;
-  if (two)
-    for (int e = lane; e < 16 * (W - 16); e += 64) bad = bad || X[(e & 15) * W + 16 + (e >> 4)] != 0.0;
+  for (int e = lane; e < 16 * (W - klow); e += 64)
+    bad = bad || ((e & 15) < W && X[(e & 15) * W + klow + (e >> 4)] != 0.0);
   if (bad) g.flag[1] = 1;
 }
 
@@ -796,8 +824,9 @@ int walls_setup(Ctx* c) {
   if ((rc = upload_vec(c, &t->umode, umode))) return rc;
   // the chunk maps of the L_k and H_k solves, one per class (not when the
   // sequential sweeps are requested)
-  const size_t nf = (size_t)chunk_count(Ny, p, false) * U * map_words(p, false),
-               nb = (size_t)chunk_count(Ny, p, true) * U * map_words(p, true);
+  const bool mx = c->fp32_primary;
+  const size_t nf = (size_t)chunk_count(Ny, p, false, mx) * U * map_words(p, false, mx),
+               nb = (size_t)chunk_count(Ny, p, true, mx) * U * map_words(p, true, mx);
   // the chunked solve also stages three right-hand sides per mode pair in
   // LDS (2 * 3 * (Ny + 32) complex values), which must fit in 64 KiB
   const bool maps_fit = nf < (1ull << 28) && nb < (1ull << 28) &&
@@ -819,6 +848,7 @@ int walls_setup(Ctx* c) {
     gs.ku = ku;
     gs.rows = rows;
     gs.U = U;
+    gs.mx = mx;
     gs.W1 = d1.width;
     gs.W2 = d2.width;
     gs.d1w = t->d1w;
@@ -857,8 +887,8 @@ int walls_setup(Ctx* c) {
       for (double** m : {&t->lk_bmap, &t->hk_bmap})
         if (!(*m = static_cast<double*>(c->alloc(nb * sizeof(double)))))
           return c->fail(DNSMI_ENOMEM, "device allocation failed");
-      hipLaunchKernelGGL(k_setup_maps, dim3(std::max(chunk_count(Ny, p, false), chunk_count(Ny, p, true)), U, 4), dim3(64), 0, nullptr, gs, t->lk_fmap, t->lk_bmap,
-                         t->hk_fmap, t->hk_bmap);
+      hipLaunchKernelGGL(k_setup_maps, dim3(std::max(chunk_count(Ny, p, false, mx), chunk_count(Ny, p, true, mx)), U, 4),
+                         dim3(64), 0, nullptr, gs, t->lk_fmap, t->lk_bmap, t->hk_fmap, t->hk_bmap);
       if ((rc = check_launch(c, "setup_maps"))) return rc;
     }
     const long long nab = (long long)Ny * rows * M;
@@ -974,8 +1004,8 @@ int walls_setup(Ctx* c) {
           auto lpiv = [&](int j) { return lk_piv[(size_t)j * M + m]; };
           auto hraw = [&](int r, int j) { return hk_ab[((size_t)j * rows + r) * M + m]; };
           auto hpiv = [&](int j) { return hk_piv[(size_t)j * M + m]; };
-          const bool a = chunk_maps(Ny, p, u, U, lraw, lpiv, lf.data(), lb.data());
-          const bool b = chunk_maps(Ny, p, u, U, hraw, hpiv, hf.data(), hb.data());
+          const bool a = chunk_maps(Ny, p, mx, u, U, lraw, lpiv, lf.data(), lb.data());
+          const bool b = chunk_maps(Ny, p, mx, u, U, hraw, hpiv, hf.data(), hb.data());
           if (!a || !b) ok[w] = 0;
         }
       };
@@ -1312,14 +1342,38 @@ __device__ __forceinline__ cx<double> imm_fhat_at(const ImmArgs& a, const Weight
   return wall ? cx<double>{0, 0} : cx<double>{(idt * d.x + dn.x) + g * lkd.x, (idt * d.y + dn.y) + g * lkd.y};
 }
 
-// R_c at row y for the three components (phase 3), zero on the walls; pp =
-// the p_P row, ur = the rows of u^n (component c at ur + c ld), nc = c N_j +
-// (1 - c) N_n at y.
+// A mixed context's f_hat at row y: N_j's and N_n's divergences apart and
+// combined last, d / dt a division.  nj1 and nn1 are the y rows of N_j and
+// N_n, n = {N_j x, N_j z, N_n x, N_n z} at y.
 template <int PO>
+__device__ __forceinline__ cx<double> imm_fhat_mx_at(const ImmArgs& a, const Weights<PO + 1>& d1,
+                                                     const Weights<PO + 2>& d2, const cx<double>* dh,
+                                                     const cx<double>* nj1, const cx<double>* nn1,
+                                                     const cx<double> (&n)[4], double kx, double kz, double k2,
+                                                     int y) {
+  const bool wall = y <= 0 || y >= a.Ny - 1;
+  const double dt = a.dt, cc = a.c, g = (1 - a.c) * a.nu;
+  const cx<double> d = dh[y];
+  const cx<double> dvj = d1(nj1), dvn = d1(nn1);
+  const cx<double> aj = ikm(kx, n[0]), cj = ikm(kz, n[1]), an = ikm(kx, n[2]), cn = ikm(kz, n[3]);
+  const cx<double> divj = {(aj.x + dvj.x) + cj.x, (aj.y + dvj.y) + cj.y};
+  const cx<double> divn = {(an.x + dvn.x) + cn.x, (an.y + dvn.y) + cn.y};
+  const cx<double> d2d = d2(dh);
+  const cx<double> lkd = {d2d.x - k2 * d.x, d2d.y - k2 * d.y};
+  return wall ? cx<double>{0, 0}
+              : cx<double>{((d.x / dt + cc * divj.x) + (1 - cc) * divn.x) + g * lkd.x,
+                           ((d.y / dt + cc * divj.y) + (1 - cc) * divn.y) + g * lkd.y};
+}
+
+// R_c at row y for the three components (phase 3), zero on the walls; pp =
+// the p_P row, ur = the rows of u^n (component c at ur + c ld); nc = c N_j +
+// (1 - c) N_n at y, or in a mixed context (MX) N_j there and nn = N_n, added
+// one by one.
+template <int PO, bool MX>
 __device__ __forceinline__ void imm_r_at(const ImmArgs& a, const Weights<PO + 1>& d1, const Weights<PO + 2>& d2,
                                          const cx<double>* pp, const cx<double>* ur, int ld,
-                                         const cx<double> (&nc)[3], double kx, double kz, double k2, int y,
-                                         cx<double> (&r)[3]) {
+                                         const cx<double> (&nc)[3], const cx<double> (&nn)[3], double kx, double kz,
+                                         double k2, int y, cx<double> (&r)[3]) {
   const bool wall = y <= 0 || y >= a.Ny - 1;
   const double idt = 1.0 / a.dt, g = (1.0 - a.c) * a.nu;
   const cx<double> p = pp[y];
@@ -1331,7 +1385,12 @@ __device__ __forceinline__ void imm_r_at(const ImmArgs& a, const Weights<PO + 1>
     const cx<double> du = d2(unc);
     const cx<double> l = {du.x - k2 * u.x, du.y - k2 * u.y};
     const cx<double> hm = {idt * u.x + g * l.x, idt * u.y + g * l.y};
-    r[c] = wall ? cx<double>{0, 0} : cx<double>{(hm.x - dpp[c].x) + nc[c].x, (hm.y - dpp[c].y) + nc[c].y};
+    if constexpr (MX)
+      r[c] = {((hm.x - dpp[c].x) + a.c * nc[c].x) + (1 - a.c) * nn[c].x,
+              ((hm.y - dpp[c].y) + a.c * nc[c].y) + (1 - a.c) * nn[c].y};
+    else
+      r[c] = {(hm.x - dpp[c].x) + nc[c].x, (hm.y - dpp[c].y) + nc[c].y};
+    if (wall) r[c] = {0, 0};
   }
 }
 
@@ -1381,11 +1440,11 @@ __device__ __forceinline__ double imm_assemble_at(const ImmArgs& a, int m, size_
 
 // Phase 1 (flows/plane_couette.py:427-445): d_hat^n into LDS, then f_hat
 // (zero on the walls) -> V_F.
-template <int PO>
+template <int PO, bool MX>
 __global__ void __launch_bounds__(kImmT) k_imm_fhat(ImmArgs a) {
   if (a.act && *a.act == 0) return;
-  // LDS: d_hat, then the y rows of u^n and c N_j + (1 - c) N_n (the D1
-  // stencils' operands, read once from HBM)
+  // LDS: d_hat, then the y rows of u^n and c N_j + (1 - c) N_n, or N_j and
+  // N_n (the D1 stencils' operands, read once from HBM)
   extern __shared__ cx<double> dh[];
   const int m = blockIdx.x, Ny = a.Ny;
   const size_t comp = (size_t)a.M * Ny, row = (size_t)m * Ny;
@@ -1393,18 +1452,32 @@ __global__ void __launch_bounds__(kImmT) k_imm_fhat(ImmArgs a) {
   const double k2 = kx * kx + kz * kz;
   cx<double>* un1 = dh + Ny;
   cx<double>* nc1 = dh + 2 * Ny;
+  [[maybe_unused]] cx<double>* nn1 = dh + 3 * Ny;
   for (int y = threadIdx.x; y < Ny; y += blockDim.x) {
     un1[y] = a.un[comp + row + y];
-    nc1[y] = imm_n_at(a, comp + row + y);
+    if constexpr (MX) {
+      nc1[y] = a.nj[comp + row + y];
+      nn1[y] = a.nn[comp + row + y];
+    } else {
+      nc1[y] = imm_n_at(a, comp + row + y);
+    }
   }
   __syncthreads();
   for (int y = threadIdx.x; y < Ny; y += blockDim.x)
     dh[y] = imm_dhat_at<PO>(Weights<PO + 1>(a.d1w, Ny, y), un1, a.un[row + y], a.un[2 * comp + row + y], kx, kz);
   __syncthreads();
   cx<double>* f = svec(a, V_F, m);
-  for (int y = threadIdx.x; y < Ny; y += blockDim.x)
-    f[y * VS] = imm_fhat_at<PO>(a, Weights<PO + 1>(a.d1w, Ny, y), Weights<PO + 2>(a.d2w, Ny, y), dh, nc1,
-                                imm_n_at(a, row + y), imm_n_at(a, 2 * comp + row + y), kx, kz, k2, y);
+  for (int y = threadIdx.x; y < Ny; y += blockDim.x) {
+    const Weights<PO + 1> d1(a.d1w, Ny, y);
+    const Weights<PO + 2> d2(a.d2w, Ny, y);
+    if constexpr (MX) {
+      const cx<double> n[4] = {a.nj[row + y], a.nj[2 * comp + row + y], a.nn[row + y], a.nn[2 * comp + row + y]};
+      f[y * VS] = imm_fhat_mx_at<PO>(a, d1, d2, dh, nc1, nn1, n, kx, kz, k2, y);
+    } else {
+      f[y * VS] = imm_fhat_at<PO>(a, d1, d2, dh, nc1, imm_n_at(a, row + y), imm_n_at(a, 2 * comp + row + y), kx, kz,
+                                  k2, y);
+    }
+  }
 }
 
 // Phases 2 and 4: solve ab x = rhs per (mode, right-hand side r =
@@ -1562,24 +1635,24 @@ __device__ __forceinline__ void wave_sync() {
 // chunk's window has behind its direction's end, the next vector's first ones
 // serving the one before.  Vector v starts at v ld + pad; ld = 4 mod 16 keeps
 // the columns of a wavefront's reads (four rows of each) on different banks.
-__host__ __device__ inline int chunk_pad(int Ny, int p) {
-  const int f = 16 * chunk_tiles(p, false) - 1 - (Ny - 1) % chunk_rows(p, false);
-  const int b = 16 * chunk_tiles(p, true) - 1 - (Ny - 1) % chunk_rows(p, true);
+__host__ __device__ inline int chunk_pad(int Ny, int p, bool mx) {
+  const int f = chunk_span(p, false, mx) - 1 - (Ny - 1) % chunk_rows(p, false, mx);
+  const int b = chunk_span(p, true, mx) - 1 - (Ny - 1) % chunk_rows(p, true, mx);
   return f > b ? f : b;
 }
-__host__ __device__ inline int chunk_ld(int Ny, int p) { return (Ny + chunk_pad(Ny, p) + 11) / 16 * 16 + 4; }
-__host__ __device__ inline int chunk_lds(int Ny, int p, int vectors) {
-  return vectors * chunk_ld(Ny, p) + chunk_pad(Ny, p);
+__host__ __device__ inline int chunk_ld(int Ny, int p, bool mx) { return (Ny + chunk_pad(Ny, p, mx) + 11) / 16 * 16 + 4; }
+__host__ __device__ inline int chunk_lds(int Ny, int p, bool mx, int vectors) {
+  return vectors * chunk_ld(Ny, p, mx) + chunk_pad(Ny, p, mx);
 }
 // Zeros over all rows that are no vector's.
-__device__ __forceinline__ void chunk_zero(cx<double>* lds, int Ny, int p, int vectors) {
-  const int pad = chunk_pad(Ny, p), gap = chunk_ld(Ny, p) - Ny;
+__device__ __forceinline__ void chunk_zero(cx<double>* lds, int Ny, int p, bool mx, int vectors) {
+  const int pad = chunk_pad(Ny, p, mx), ld = chunk_ld(Ny, p, mx), gap = ld - Ny;
   for (int v = 0; v < vectors; ++v)
     for (int i = threadIdx.x; i < gap; i += blockDim.x) {
-      const int row = v * chunk_ld(Ny, p) + (i < pad ? i : Ny + i);
+      const int row = v * ld + (i < pad ? i : Ny + i);
       lds[row] = cx<double>{0, 0};
     }
-  for (int i = threadIdx.x; i < pad; i += blockDim.x) lds[vectors * chunk_ld(Ny, p) + i] = cx<double>{0, 0};
+  for (int i = threadIdx.x; i < pad; i += blockDim.x) lds[vectors * ld + i] = cx<double>{0, 0};
 }
 
 // Chunk c's operands e, e + 1 of this lane (chunks past the last repeat it).
@@ -1591,16 +1664,16 @@ struct MapChunk {
 };
 
 // Chunks of maps in registers, loaded that many less one ahead: eight words a
-// lane each in one-tile windows, 24 in two-tile ones.
-template <int PO, bool BACK>
+// lane each in one-tile windows, 20 to 24 in two-tile ones.
+template <int PO, bool BACK, bool MX>
 struct ChunkMaps {
-  static constexpr int R = chunk_tiles(PO, BACK) == 1 ? 4 : 3, N = map_operands(PO, BACK);
+  static constexpr int R = chunk_tiles(PO, BACK, MX) == 1 ? 4 : 3, N = map_operands(PO, BACK, MX);
   double f[R][N];
   // the first R - 1 chunks'
   __device__ __forceinline__ void start(const double* __restrict__ map, int U, int u, int lane, int Ny) {
 #pragma unroll
     for (int q = 0; q < R - 1; ++q) {
-      const MapChunk m(map, U, u, map_words(PO, BACK), q, chunk_count(Ny, PO, BACK), lane);
+      const MapChunk m(map, U, u, map_words(PO, BACK, MX), q, chunk_count(Ny, PO, BACK, MX), lane);
 #pragma unroll
       for (int e = 0; e < N / 2; ++e) {
         const double2 v = m(e);
@@ -1623,15 +1696,18 @@ struct ChunkMaps {
 // kept ones) before the first: a result's latency passes behind products that
 // do not need it.  Behind each product (64 cycles of the matrix core) stands
 // its share of the loads and stores, pinned there: in front of the products
-// they cost half as much again.
-template <int PO, bool BACK>
+// they cost half as much again.  A mixed context's k steps are in ascending
+// order (chunk_tiles).
+template <int PO, bool BACK, bool MX>
 __device__ __forceinline__ void chunk_chain(const double* __restrict__ map, int U, int u, int lane, int Ny, double* pc,
-                                            ChunkMaps<PO, BACK>& maps) {
-  constexpr int TILES = chunk_tiles(PO, BACK), B = chunk_rows(PO, BACK), KEEP = BACK ? 2 * PO : PO;
-  constexpr int R = ChunkMaps<PO, BACK>::R, N = ChunkMaps<PO, BACK>::N;
-  constexpr int WR = 4 * TILES, KR = (KEEP + 3) / 4, BR = B / 4, S = BACK ? -1 : 1;
+                                            ChunkMaps<PO, BACK, MX>& maps) {
+  constexpr int TILES = chunk_tiles(PO, BACK, MX), B = chunk_rows(PO, BACK, MX), KEEP = chunk_keep(PO, BACK);
+  constexpr int R = ChunkMaps<PO, BACK, MX>::R, N = ChunkMaps<PO, BACK, MX>::N;
+  constexpr int NH = high_operands(PO, BACK, MX), NL = low_operands(PO, BACK, MX);
+  constexpr int WR = chunk_span(PO, BACK, MX) / 4, KR = (KEEP + 3) / 4, BR = B / 4, S = BACK ? -1 : 1;
   static_assert(KR + BR == WR, "kept and new rows fill the window's registers");
-  const int g = lane >> 4, nC = chunk_count(Ny, PO, BACK);
+  static_assert(NH <= WR && NL <= WR && BR <= NH + NL && N / 2 <= NH + NL, "each product's operand, load and store");
+  const int g = lane >> 4, nC = chunk_count(Ny, PO, BACK, MX);
   double* pg = pc + 2 * ((BACK ? Ny - 1 : 0) + S * g);  // this lane group's row of the first chunk
   double w[WR], done[BR];                               // the window; chunk c - 1's results
 #pragma unroll
@@ -1639,7 +1715,7 @@ __device__ __forceinline__ void chunk_chain(const double* __restrict__ map, int 
 #pragma unroll
   for (int i = 0; i < BR; ++i) done[i] = 0.0;
   auto step = [&](int c, double(&fc)[N], double(&pf)[N]) {
-    const MapChunk m(map, U, u, map_words(PO, BACK), c + R - 1, nC, lane);
+    const MapChunk m(map, U, u, map_words(PO, BACK, MX), c + R - 1, nC, lane);
     // (the last chunk asks for its own rows again; chunk 0 stores zeros over
     // rows that the window holds and chunk 1 stores)
     double* in = pg + 2 * S * min(c + 1, nC - 1) * B;
@@ -1649,11 +1725,11 @@ __device__ __forceinline__ void chunk_chain(const double* __restrict__ map, int 
 #pragma unroll
     for (int i = 0; i < TILES; ++i) acc[i] = wd4{0, 0, 0, 0};
 #pragma unroll
-    for (int e = 0; e < N; ++e) {
+    for (int e = 0; e < NH + NL; ++e) {
       // product e: tile, k step q, operand of the map
-      const int tile = TILES == 1 || e >= 8 ? 0 : 1, K = TILES == 1 || e >= 8 ? 4 : 8;
-      const int i = TILES == 2 && e >= 8 ? e - 8 : e, kr = KR < K ? KR : 0, q = i < K - kr ? kr + i : i - (K - kr);
-      acc[tile] = __builtin_amdgcn_mfma_f64_16x16x4f64(fc[TILES == 2 && e >= 8 ? 8 + q : q], w[q], acc[tile], 0, 0, 0);
+      const int tile = e < NH ? 1 : 0, K = tile ? NH : NL, i = tile ? e : e - NH;
+      const int kr = !MX && KR < K ? KR : 0, q = i < K - kr ? kr + i : i - (K - kr);
+      acc[tile] = __builtin_amdgcn_mfma_f64_16x16x4f64(fc[tile ? q : NH + q], w[q], acc[tile], 0, 0, 0);
       if (e < N / 2) {
         const double2 v = m(e);
         pf[2 * e] = v.x;
@@ -1688,15 +1764,15 @@ __device__ __forceinline__ void chunk_chain(const double* __restrict__ map, int 
 
 // Band solve of this wavefront's columns, in place; maps: the forward maps,
 // started.
-template <int PO>
+template <int PO, bool MX>
 __device__ __forceinline__ void chunk_solve(const double* __restrict__ fmap, const double* __restrict__ bmap, int U,
-                                            int u, int lane, int Ny, double* pc, ChunkMaps<PO, false>& maps) {
-  ChunkMaps<PO, true> back;
+                                            int u, int lane, int Ny, double* pc, ChunkMaps<PO, false, MX>& maps) {
+  ChunkMaps<PO, true, MX> back;
   back.start(bmap, U, u, lane, Ny);
   wave_sync();
-  chunk_chain<PO, false>(fmap, U, u, lane, Ny, pc, maps);
+  chunk_chain<PO, false, MX>(fmap, U, u, lane, Ny, pc, maps);
   wave_sync();
-  chunk_chain<PO, true>(bmap, U, u, lane, Ny, pc, back);
+  chunk_chain<PO, true, MX>(bmap, U, u, lane, Ny, pc, back);
   wave_sync();
 }
 
@@ -1726,22 +1802,22 @@ __device__ __forceinline__ int2 sched_mode(const int2* __restrict__ sched, int s
   return mu;
 }
 
-template <int PO, int NR>
+template <int PO, int NR, bool MX>
 __global__ void __launch_bounds__(64, 2)
     k_band_chunks(ImmArgs a, const double* __restrict__ fmap, const double* __restrict__ bmap,
                   const int2* __restrict__ sched, int U, int vin, int vout) {
   if (a.act && *a.act == 0) return;
-  extern __shared__ cx<double> lds[];  // chunk_lds(Ny, PO, 2 NR): [2][NR][ld]
-  const int Ny = a.Ny, M = a.M, ld = chunk_ld(Ny, PO), lane = threadIdx.x;
-  cx<double>* sh = lds + chunk_pad(Ny, PO);
+  extern __shared__ cx<double> lds[];  // chunk_lds(Ny, PO, MX, 2 NR): [2][NR][ld]
+  const int Ny = a.Ny, M = a.M, ld = chunk_ld(Ny, PO, MX), lane = threadIdx.x;
+  cx<double>* sh = lds + chunk_pad(Ny, PO, MX);
   const int item = xcd_block(blockIdx.x, gridDim.x);
   const size_t vs = (size_t)M * Ny;  // between work vectors (VS = 1: rows contiguous)
   bool live[2];
   int2 mu[2];
   for (int h = 0; h < 2; ++h) mu[h] = sched_mode(sched, 2 * item + h, live[h]);
-  ChunkMaps<PO, false> maps;
+  ChunkMaps<PO, false, MX> maps;
   maps.start(fmap, U, mu[0].y, lane, Ny);
-  chunk_zero(lds, Ny, PO, 2 * NR);
+  chunk_zero(lds, Ny, PO, MX, 2 * NR);
   // the right-hand sides, all in flight (rows past the end load and store the
   // last one again)
   for (int i0 = 0; i0 < Ny; i0 += 4 * 64) {
@@ -1756,7 +1832,7 @@ __global__ void __launch_bounds__(64, 2)
 #pragma unroll
       for (int r = 0; r < 2 * NR; ++r) sh[r * ld + min(i0 + q * 64 + lane, Ny - 1)] = v[q][r];
   }
-  chunk_solve<PO>(fmap, bmap, U, mu[0].y, lane, Ny, chunk_column<NR>(sh, NR * ld, ld, lane), maps);
+  chunk_solve<PO, MX>(fmap, bmap, U, mu[0].y, lane, Ny, chunk_column<NR>(sh, NR * ld, ld, lane), maps);
   for (int i = lane; i < Ny; i += 64)
 #pragma unroll
     for (int r = 0; r < 2 * NR; ++r)
@@ -1782,42 +1858,51 @@ __global__ void __launch_bounds__(64, 2)
 // was the fastest before: 128 x 256 x 128, p = 6, five launches 623 us, so
 // 296 us; 64 x 128 x 64, p = 4, two launches (solve and parallel phases by
 // each wavefront) 68 us, so 27 us; 48 x 65 x 32, p = 4: 35 us, so 12 us.
+// Mixed contexts (MX; chunk_tiles): 128 x 256 x 128, p = 6, 563 us, so 336 us.
 constexpr int kImmRows = 4;       // LDS rows per mode
 constexpr int kImmFusedNy = 278;  // largest Ny of the fused form
 
-template <int PO, int YP>
+template <int PO, int YP, bool MX>
 __global__ void __launch_bounds__(128, 2)
     k_imm_fused(ImmArgs a, const double* __restrict__ lf, const double* __restrict__ lb,
                 const double* __restrict__ hf, const double* __restrict__ hb, const int2* __restrict__ sched, int U) {
   if (a.act && *a.act == 0) return;
-  extern __shared__ cx<double> lds[];  // chunk_lds(Ny, PO, 2 kImmRows): [2][kImmRows][ld]
-  const int Ny = a.Ny, M = a.M, ld = chunk_ld(Ny, PO), hs = kImmRows * ld;
-  cx<double>* sh = lds + chunk_pad(Ny, PO);
+  extern __shared__ cx<double> lds[];  // chunk_lds(Ny, PO, MX, 2 kImmRows): [2][kImmRows][ld]
+  const int Ny = a.Ny, M = a.M, ld = chunk_ld(Ny, PO, MX), hs = kImmRows * ld;
+  cx<double>* sh = lds + chunk_pad(Ny, PO, MX);
   const int lane = threadIdx.x & 63, half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int item = xcd_block(blockIdx.x, gridDim.x);
   const bool solver = half == 0;
   bool live;
   const int2 mu = sched_mode(sched, 2 * item + half, live);
   const int m = mu.x, u = __builtin_amdgcn_readfirstlane(mu.y);
-  ChunkMaps<PO, false> maps;
+  ChunkMaps<PO, false, MX> maps;
   if (solver) maps.start(lf, U, u, lane, Ny);
-  chunk_zero(lds, Ny, PO, 2 * kImmRows);
+  chunk_zero(lds, Ny, PO, MX, 2 * kImmRows);
   cx<double>* r0 = sh + half * hs;
   cx<double>*r1 = r0 + ld, *r2 = r0 + 2 * ld, *r3 = r0 + 3 * ld;
   const size_t comp = (size_t)M * Ny, row = (size_t)m * Ny;
   const double kx = a.mkx[m], kz = a.mkz[m];
   const double k2 = kx * kx + kz * kz;
-  // phase 1: u^n_y in r1, c N_j + (1 - c) N_n (y) in r0, d_hat in r2, f_hat in r3
-  cx<double> ux[YP], uz[YP], nc[YP][3];
+  // phase 1: u^n_y in r1, c N_j + (1 - c) N_n (y) in r0, d_hat in r2, f_hat in
+  // r3; mixed: N_j (y) in r0, N_n (y) in r3 until f_hat replaces it, and the
+  // fields are read again where the other components are needed
+  cx<double> ux[YP], uz[YP];
+  [[maybe_unused]] cx<double> nc[YP][3], fh[YP];
 #pragma unroll
   for (int j = 0; j < YP; ++j) {
     const int y = min(lane + 64 * j, Ny - 1);
     ux[j] = a.un[row + y];
     uz[j] = a.un[2 * comp + row + y];
     r1[y] = a.un[comp + row + y];
+    if constexpr (MX) {
+      r0[y] = a.nj[comp + row + y];
+      r3[y] = a.nn[comp + row + y];
+    } else {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) nc[j][c] = imm_n_at(a, c * comp + row + y);
-    r0[y] = nc[j][1];
+      for (int c = 0; c < 3; ++c) nc[j][c] = imm_n_at(a, c * comp + row + y);
+      r0[y] = nc[j][1];
+    }
   }
   // weights of G rows at a time: all their loads in flight, within the registers
   constexpr int G = YP < 2 ? YP : 2;
@@ -1837,17 +1922,27 @@ __global__ void __launch_bounds__(128, 2)
   for (int j0 = 0; j0 < YP; j0 += G) {
     Weights<PO + 1> d1[G];
     Weights<PO + 2> d2[G];
+    [[maybe_unused]] cx<double> n[G][4];
 #pragma unroll
     for (int j = 0; j < G && j0 + j < YP; ++j) {
       int y = min(lane + 64 * (j0 + j), Ny - 1);
       if (YP > G) y = opaque(y);
       d1[j] = Weights<PO + 1>(a.d1w, Ny, y);
       d2[j] = Weights<PO + 2>(a.d2w, Ny, y);
+      if constexpr (MX) {
+        n[j][0] = a.nj[row + y];
+        n[j][1] = a.nj[2 * comp + row + y];
+        n[j][2] = a.nn[row + y];
+        n[j][3] = a.nn[2 * comp + row + y];
+      }
     }
 #pragma unroll
     for (int j = 0; j < G && j0 + j < YP; ++j) {
       const int y = min(lane + 64 * (j0 + j), Ny - 1);
-      r3[y] = imm_fhat_at<PO>(a, d1[j], d2[j], r2, r0, nc[j0 + j][0], nc[j0 + j][2], kx, kz, k2, y);
+      if constexpr (MX)
+        fh[j0 + j] = imm_fhat_mx_at<PO>(a, d1[j], d2[j], r2, r0, r3, n[j], kx, kz, k2, y);
+      else
+        r3[y] = imm_fhat_at<PO>(a, d1[j], d2[j], r2, r0, nc[j0 + j][0], nc[j0 + j][2], kx, kz, k2, y);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -1858,11 +1953,12 @@ __global__ void __launch_bounds__(128, 2)
     const int y = min(lane + 64 * j, Ny - 1);
     r0[y] = ux[j];
     r2[y] = uz[j];
+    if constexpr (MX) r3[y] = fh[j];
   }
   __syncthreads();
   // phase 2: p_P in r3
   if (solver) {
-    chunk_solve<PO>(lf, lb, U, u, lane, Ny, chunk_column<1>(sh + 3 * ld, hs, ld, lane), maps);
+    chunk_solve<PO, MX>(lf, lb, U, u, lane, Ny, chunk_column<1>(sh + 3 * ld, hs, ld, lane), maps);
     maps.start(hf, U, u, lane, Ny);
   }
   // phase 3: R_c in r0, r1, r2 (through registers: the stencils read them)
@@ -1872,17 +1968,26 @@ __global__ void __launch_bounds__(128, 2)
     for (int j0 = 0; j0 < YP; j0 += G) {
       Weights<PO + 1> e1[G];
       Weights<PO + 2> e2[G];
+      [[maybe_unused]] cx<double> nj[G][3], nn[G][3];
 #pragma unroll
       for (int j = 0; j < G && j0 + j < YP; ++j) {
         // opaque: else phase 1's weights wait in registers through the solve
         const int y = opaque(min(lane + 64 * (j0 + j), Ny - 1));
         e1[j] = Weights<PO + 1>(a.d1w, Ny, y);
         e2[j] = Weights<PO + 2>(a.d2w, Ny, y);
+        if constexpr (MX) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            nj[j][c] = a.nj[c * comp + row + y];
+            nn[j][c] = a.nn[c * comp + row + y];
+          }
+        }
       }
       if (j0 == 0) __syncthreads();  // p_P is there
 #pragma unroll
       for (int j = 0; j < G && j0 + j < YP; ++j)
-        imm_r_at<PO>(a, e1[j], e2[j], r3, r0, ld, nc[j0 + j], kx, kz, k2, min(lane + 64 * (j0 + j), Ny - 1), r[j0 + j]);
+        imm_r_at<PO, MX>(a, e1[j], e2[j], r3, r0, ld, MX ? nj[j] : nc[j0 + j], nn[j], kx, kz, k2,
+                         min(lane + 64 * (j0 + j), Ny - 1), r[j0 + j]);
       __builtin_amdgcn_sched_barrier(0);
     }
     wave_sync();
@@ -1893,7 +1998,7 @@ __global__ void __launch_bounds__(128, 2)
   }
   __syncthreads();
   // phase 4: the arbitrary velocity in r0, r1, r2
-  if (solver) chunk_solve<PO>(hf, hb, U, u, lane, Ny, chunk_column<3>(sh, hs, ld, lane), maps);
+  if (solver) chunk_solve<PO, MX>(hf, hb, U, u, lane, Ny, chunk_column<3>(sh, hs, ld, lane), maps);
   // phase 5, its operands asked for before the barrier (the wavefront that
   // does not solve has them by then)
   double4 vq[YP];
@@ -1923,7 +2028,7 @@ __global__ void __launch_bounds__(128, 2)
 
 // Phase 3 (flows/plane_couette.py:449-472): R_c for the three components
 // (zero on the walls) -> V_R + c, with the pressure row in LDS.
-template <int PO>
+template <int PO, bool MX>
 __global__ void __launch_bounds__(kImmT) k_imm_rc(ImmArgs a) {
   if (a.act && *a.act == 0) return;
   // LDS: the p_P row, then the rows of u^n (the D2 stencils' operands)
@@ -1941,10 +2046,19 @@ __global__ void __launch_bounds__(kImmT) k_imm_rc(ImmArgs a) {
   }
   __syncthreads();
   for (int y = threadIdx.x; y < Ny; y += blockDim.x) {
-    cx<double> nc[3], r[3];
+    cx<double> nc[3], nn[3], r[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) nc[c] = imm_n_at(a, c * comp + row + y);
-    imm_r_at<PO>(a, Weights<PO + 1>(a.d1w, Ny, y), Weights<PO + 2>(a.d2w, Ny, y), pp, ur, Ny, nc, kx, kz, k2, y, r);
+    for (int c = 0; c < 3; ++c) {
+      const size_t e = c * comp + row + y;
+      if constexpr (MX) {
+        nc[c] = a.nj[e];
+        nn[c] = a.nn[e];
+      } else {
+        nc[c] = imm_n_at(a, e);
+      }
+    }
+    imm_r_at<PO, MX>(a, Weights<PO + 1>(a.d1w, Ny, y), Weights<PO + 2>(a.d2w, Ny, y), pp, ur, Ny, nc, nn, kx, kz, k2,
+                     y, r);
 #pragma unroll
     for (int c = 0; c < 3; ++c) svec(a, V_R + c, m)[y * VS] = r[c];
   }
@@ -2098,6 +2212,46 @@ int walls_guess_rhs(Ctx* c, const double* state, double* rhs, hipStream_t s) {
   return walls_rhs_mode(c, state, rhs, s, EV_PLAIN);
 }
 
+// The launches of one step; MX: a mixed context's.
+template <int PO, bool MX>
+static int launch_imm(Ctx* c, const ImmArgs& a, hipStream_t s) {
+  WallTables* t = c->wt;
+  const int Ny = t->Ny;
+  const size_t row = (size_t)Ny * sizeof(cx<double>);
+  const dim3 gm(t->M), gc(t->items);
+  if (c->imm_fused && !c->sweep_seq) {
+    if (Ny > kImmFusedNy) return c->fail(DNSMI_EINVAL, "imm: ny too large for the fused form");
+    const size_t lds = (size_t)chunk_lds(Ny, PO, MX, 2 * kImmRows) * sizeof(cx<double>);
+    auto fused = [&](auto yp) {
+      hipLaunchKernelGGL((k_imm_fused<PO, decltype(yp)::value, MX>), gc, dim3(128), lds, s, a, t->lk_fmap, t->lk_bmap,
+                         t->hk_fmap, t->hk_bmap, t->sched, t->U);
+    };
+    if (Ny <= 64) fused(std::integral_constant<int, 1>{});
+    else if (Ny <= 128) fused(std::integral_constant<int, 2>{});
+    else if (Ny <= 256) fused(std::integral_constant<int, 4>{});
+    else fused(std::integral_constant<int, 5>{});
+    return DNSMI_OK;
+  }
+  // solves of nr right-hand sides per mode
+  auto solve = [&](auto nr, const double* ab, const int* piv, const double* fmap, const double* bmap, int vin,
+                   int vout) {
+    constexpr int NR = decltype(nr)::value;
+    if (c->sweep_seq)
+      hipLaunchKernelGGL(k_band_sweeps<PO>, dim3((t->M + kSweepLanes - 1) / kSweepLanes, NR), dim3(kSweepLanes), 0, s,
+                         a, ab, piv, vin, (int)V_T, vout);
+    else  // per workgroup two modes' vectors in LDS
+      hipLaunchKernelGGL((k_band_chunks<PO, NR, MX>), gc, dim3(64),
+                         (size_t)chunk_lds(Ny, PO, MX, 2 * NR) * sizeof(cx<double>), s, a, fmap, bmap, t->sched, t->U,
+                         vin, vout);
+  };
+  hipLaunchKernelGGL((k_imm_fhat<PO, MX>), gm, dim3(kImmT), (MX ? 4 : 3) * row, s, a);
+  solve(std::integral_constant<int, 1>{}, t->lk_ab, t->lk_piv, t->lk_fmap, t->lk_bmap, (int)V_F, (int)V_P);
+  hipLaunchKernelGGL((k_imm_rc<PO, MX>), gm, dim3(kImmT), 4 * row, s, a);
+  solve(std::integral_constant<int, 3>{}, t->hk_ab, t->hk_piv, t->hk_fmap, t->hk_bmap, (int)V_R, (int)V_R);
+  hipLaunchKernelGGL(k_imm_final<PO>, gm, dim3(kImmT), 0, s, a);
+  return DNSMI_OK;
+}
+
 static int walls_imm(Ctx* c, const double* un, const double* uj, const double* nn,
                      const double* nj, double* out, double* corr, double* err, hipStream_t s) {
   WallTables* t = c->wt;
@@ -2134,57 +2288,20 @@ static int walls_imm(Ctx* c, const double* un, const double* uj, const double* n
   {
     if (!c->sweep_seq && !t->lk_fmap) return c->fail(DNSMI_EINVAL, "imm: chunk maps not built");
     ProfScope ps(c, KID_W_IMM, s);
-    const size_t lds = (size_t)t->Ny * sizeof(cx<double>);
-    const dim3 gm(t->M), gs((t->M + kSweepLanes - 1) / kSweepLanes, 1),
-        gs3((t->M + kSweepLanes - 1) / kSweepLanes, 3), gc(t->items);
-    // chunked solves: per workgroup two modes' vectors
-    const size_t lds_c1 = (size_t)chunk_lds(t->Ny, t->p, 2) * sizeof(cx<double>);
-    const size_t lds_c3 = (size_t)chunk_lds(t->Ny, t->p, 6) * sizeof(cx<double>);
-    if (4 * lds > 65536 || (!c->sweep_seq && (size_t)2 * 3 * (t->Ny + 32) * sizeof(cx<double>) > 65536))
+    if (4 * (size_t)t->Ny * sizeof(cx<double>) > 65536 ||
+        (!c->sweep_seq && (size_t)2 * 3 * (t->Ny + 32) * sizeof(cx<double>) > 65536))
       return c->fail(DNSMI_EINVAL, "imm: ny too large for the per-mode LDS rows");
-    if (c->imm_fused && !c->sweep_seq) {
-      if (t->Ny > kImmFusedNy) return c->fail(DNSMI_EINVAL, "imm: ny too large for the fused form");
-      const size_t lds_f = (size_t)chunk_lds(t->Ny, t->p, 2 * kImmRows) * sizeof(cx<double>);
-#define IMMF(PO, YP)                                                                                      \
-  hipLaunchKernelGGL((k_imm_fused<PO, YP>), gc, dim3(128), lds_f, s, a, t->lk_fmap, t->lk_bmap, \
-                     t->hk_fmap, t->hk_bmap, t->sched, t->U)
-#define IMMFP(PO)                       \
-  case PO:                              \
-    if (t->Ny <= 64) IMMF(PO, 1);       \
-    else if (t->Ny <= 128) IMMF(PO, 2); \
-    else if (t->Ny <= 256) IMMF(PO, 4); \
-    else IMMF(PO, 5);                   \
-    break;
-      switch (t->p) {
-        IMMFP(2) IMMFP(4) IMMFP(6) IMMFP(8)
-        default: return c->fail(DNSMI_EINVAL, "fd_order");
-      }
-#undef IMMFP
-#undef IMMF
-    } else
+    int rc = DNSMI_OK;
     switch (t->p) {
-#define IMM(PO)                                                                                   \
-  case PO:                                                                                        \
-    hipLaunchKernelGGL(k_imm_fhat<PO>, gm, dim3(kImmT), 3 * lds, s, a);                           \
-    if (c->sweep_seq)                                                                             \
-      hipLaunchKernelGGL(k_band_sweeps<PO>, gs, dim3(kSweepLanes), 0, s, a, t->lk_ab, t->lk_piv,   \
-                         (int)V_F, (int)V_T, (int)V_P);                                           \
-    else                                                                                          \
-      hipLaunchKernelGGL((k_band_chunks<PO, 1>), gc, dim3(64), lds_c1, s, a, t->lk_fmap,          \
-                         t->lk_bmap, t->sched, t->U, (int)V_F, (int)V_P);                         \
-    hipLaunchKernelGGL(k_imm_rc<PO>, gm, dim3(kImmT), 4 * lds, s, a);                             \
-    if (c->sweep_seq)                                                                             \
-      hipLaunchKernelGGL(k_band_sweeps<PO>, gs3, dim3(kSweepLanes), 0, s, a, t->hk_ab, t->hk_piv, \
-                         (int)V_R, (int)V_T, (int)V_R);                                           \
-    else                                                                                          \
-      hipLaunchKernelGGL((k_band_chunks<PO, 3>), gc, dim3(64), lds_c3, s, a, t->hk_fmap,          \
-                         t->hk_bmap, t->sched, t->U, (int)V_R, (int)V_R);                         \
-    hipLaunchKernelGGL(k_imm_final<PO>, gm, dim3(kImmT), 0, s, a);                                \
+#define IMM(PO)                                                                       \
+  case PO:                                                                            \
+    rc = c->fp32_primary ? launch_imm<PO, true>(c, a, s) : launch_imm<PO, false>(c, a, s); \
     break;
       IMM(2) IMM(4) IMM(6) IMM(8)
 #undef IMM
       default: return c->fail(DNSMI_EINVAL, "fd_order");
     }
+    if (rc) return rc;
   }
   int rc = check_launch(c, "imm");
   if (rc || !err) return rc;
@@ -2406,7 +2523,7 @@ int walls_table(Ctx* c, int which, double* out, long long n) {
     case 10:
     case 11: {
       const bool back = which == 9 || which == 11;
-      const size_t words = (size_t)chunk_count(Ny, t->p, back) * U * map_words(t->p, back);
+      const size_t words = (size_t)chunk_count(Ny, t->p, back, c->fp32_primary) * U * map_words(t->p, back, c->fp32_primary);
       const double* src = which == 8 ? t->lk_fmap : which == 9 ? t->lk_bmap : which == 10 ? t->hk_fmap : t->hk_bmap;
       if (!src) return want(0);
       if ((rc = want((long long)words))) return rc;
@@ -2417,8 +2534,10 @@ int walls_table(Ctx* c, int which, double* out, long long n) {
       if ((rc = want(5))) return rc;
       out[4] = U;
       const double* maps[4] = {t->lk_fmap, t->lk_bmap, t->hk_fmap, t->hk_bmap};
-      for (int i = 0; i < 4; ++i)
-        out[i] = maps[i] ? (double)((size_t)chunk_count(Ny, t->p, i % 2 != 0) * U * map_words(t->p, i % 2 != 0)) : 0.0;
+      for (int i = 0; i < 4; ++i) {
+        const bool back = i % 2 != 0, mx = c->fp32_primary;
+        out[i] = maps[i] ? (double)((size_t)chunk_count(Ny, t->p, back, mx) * U * map_words(t->p, back, mx)) : 0.0;
+      }
       return DNSMI_OK;
     }
     default: return c->fail(DNSMI_EINVAL, "unknown table");
