@@ -1634,13 +1634,24 @@ static int launch_z_forward(Ctx* c, hipStream_t s) {
 
 template <typename T, int P, int TC, int MODE, bool PADY>
 static void launch_y_forward_p(Ctx* c, int nb, const YFwdArgs& a, hipStream_t s) {
-  // Three components of 16 columns that take more than half a CU's LDS leave
-  // one workgroup to it: with more workgroups than CUs nothing overlaps one's
-  // transforms with another's loads, and the serial form is the faster one.
-  // FP64 step at 128^3 (508 workgroups): 786 us serial, 789 us side by side;
-  // 64 x 128^2 (254): 449 us serial, 411 us side by side.
-  if constexpr (3 * TC * P * sizeof(cx<T>) > 80 * 1024) {
-    if (nb > kCUs) {
+  // Three components of 16 FP64 columns that take more than half a CU's LDS
+  // leave one workgroup to it: with more workgroups than CUs nothing overlaps
+  // one's transforms with another's loads, and the serial form is the faster
+  // one.  FP64 step at 128^3 (508 workgroups): 839 us serial, 865 us side by
+  // side; 64 x 128^2 (254): 437 and 415 us.  FP32 tiles leave two workgroups to
+  // a CU; from 144 rows on the serial form is the faster one where nearly all
+  // of those places are taken: mixed step at 128^3 (508) 708 and 715 us, 128 x
+  // 96 x 128 562 and 568 us from a guess, but 128 x 128 x 96 (380) 547 and 540
+  // us and 96 x 64 x 96 and 128 x 64 x 128 (285, 508; 96 rows) within 0.6 %.
+  //
+  // nb is one member's workgroups, in a batch too: the two forms sum the norm in
+  // different orders, and a member's error equals its eager run's to the bit.
+  // That costs large batches (16 x 64^3 FP64: 3446 us serial, 3480 us side by
+  // side) what it gains small ones (4 x 32^3 FP64: 315 and 294 us).
+  constexpr size_t tile = 3 * TC * P * sizeof(cx<T>);
+  constexpr bool fp64 = std::is_same<T, double>::value;
+  if constexpr (tile > (fp64 ? 80 : 50) * 1024) {
+    if (nb > (fp64 ? kCUs : kCUs * 3 / 2)) {
       launch(c, &k_y_forward_serial<T, P, TC, MODE, PADY>, &k_y_forward_serial_b<T, P, TC, MODE, PADY>, dim3(nb),
              dim3(TC * ColPlan<P>::threads), s, a);
       return;
