@@ -616,8 +616,10 @@ int pnet_forward(int din, int H, int dout, int B, const uint16_t* X, const float
 
 // A weight gradient G (M + 1 rows: the weights', then the bias's) = [P | 1]^T
 // Q over the batch, P (B, M), Q (B, N): up to `want` workgroups by splitting
-// the batch, each part at least 128 samples, as far as `room` floats of
-// scratch hold the parts (one part needs none and goes straight to G).
+// the batch into parts of equal numbers of 64-sample chunks (the last part
+// takes what is left), two chunks each at least where the batch has them, as
+// far as `room` floats of scratch hold the parts (one part needs none and goes
+// straight to G).
 struct WGrad {
   GemmArgs g;
   int blocks;
@@ -635,6 +637,10 @@ static WGrad pn_wgrad(int M, int N, int B, const uint16_t* P, const uint16_t* Q,
   if (parts > (B + 127) / 128) parts = (B + 127) / 128;
   if (parts > room / n) parts = room / n;
   if (parts < 1) parts = 1;
+  // the chunks of a part rounded up leave the last parts none: as many parts
+  // as have some (pn_tile divides the batch the same way)
+  const long long chunks = ((long long)B + kPnK - 1) / kPnK, per = (chunks + parts - 1) / parts;
+  parts = (chunks + per - 1) / per;
   r.g.M = M;
   r.g.N = N;
   r.g.K = B;
