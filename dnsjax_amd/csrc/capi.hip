@@ -96,19 +96,18 @@ int mlp_grad_static(int H, int B, const float* X, const float* T, const float* p
 long long mlp_grad_scratch(int H, int B);
 int mlp_adam(int H, float* prm, const float* g, float* m, float* v, int step, float lr,
              hipStream_t s);
-int pnet_forward(int din, int H, int dout, int B, const uint16_t* X, const float* prm, uint16_t* wb,
-                 float* wf, uint16_t* wh, float* Y, hipStream_t s);
+int pnet_forward(int din, int H, int dout, int B, const uint16_t* X, const float* prm, uint16_t* wb, uint16_t* wh,
+                 float* Y, hipStream_t s);
 int pnet_grad(int din, int H, int dout, int B, const uint16_t* X, const float* T, const float* prm,
-              uint16_t* wb, float* wf, uint16_t* wh, float* part, float* grad, float* loss,
-              hipStream_t s);
+              uint16_t* wb, float* wf, uint16_t* wh, float* grad, float* loss, hipStream_t s);
 int pnet_adam(long long P, float* prm, const float* g, float* m, float* v, int step, float lr,
               hipStream_t s);
 int pnet_features(Ctx* c, const double* nm2, const double* nm1, const double* ncur, const double* nnext,
                   const long long* modes, int ns, int din, float s_1, float s_2, float s_out, uint16_t* X,
                   float* T, hipStream_t s);
 int guess_walls_profile(Ctx* c, const double* state, double* pred, double* rhs_prev, const float* h1, float* h2,
-                        int din, int H, int dout, const float* prm, uint16_t* wb, uint16_t* X, float* wf,
-                        uint16_t* wh, float* Y, float s_1, float s_2, float s_out, hipStream_t s);
+                        int din, int H, int dout, const float* prm, uint16_t* wb, uint16_t* X, uint16_t* wh,
+                        float* Y, float s_1, float s_2, float s_out, hipStream_t s);
 int mlp_pack(int H, const float* prm, uint16_t* wb, float* bias, hipStream_t s);
 int mlp_forward(int H, const float* X, int B, const uint16_t* wb, const float* bias, float* Y,
                 hipStream_t s);
@@ -400,21 +399,21 @@ long long dnsmi_pnet_params(int din, int H, int dout) {
 }
 
 int dnsmi_pnet_grad(int din, int H, int dout, int B, const void* X, const float* T, const float* params,
-                    void* wb, float* wf, void* wh, float* part, float* grad, float* loss_dev, void* stream) {
-  if (!X || !T || !params || !wb || !wf || !wh || !part || !grad || B <= 0 || dnsmi_pnet_params(din, H, dout) < 0)
+                    void* wb, float* wf, void* wh, float* /*part*/, float* grad, float* loss_dev, void* stream) {
+  if (!X || !T || !params || !wb || !wf || !wh || !grad || B <= 0 || dnsmi_pnet_params(din, H, dout) < 0)
     return ctxfree(DNSMI_EINVAL, "pnet_grad");
   return ctxfree(dnsmi::pnet_grad(din, H, dout, B, static_cast<const uint16_t*>(X), T, params,
-                                  static_cast<uint16_t*>(wb), wf, static_cast<uint16_t*>(wh), part, grad,
-                                  loss_dev, as_stream(stream)),
+                                  static_cast<uint16_t*>(wb), wf, static_cast<uint16_t*>(wh), grad, loss_dev,
+                                  as_stream(stream)),
                  "pnet_grad");
 }
 
 int dnsmi_pnet_forward(int din, int H, int dout, int B, const void* X, const float* params, void* wb,
-                       float* wf, void* wh, float* Y, void* stream) {
-  if (!X || !params || !wb || !wf || !wh || !Y || B <= 0 || dnsmi_pnet_params(din, H, dout) < 0)
+                       float* /*wf*/, void* wh, float* Y, void* stream) {
+  if (!X || !params || !wb || !wh || !Y || B <= 0 || dnsmi_pnet_params(din, H, dout) < 0)
     return ctxfree(DNSMI_EINVAL, "pnet_forward");
   return ctxfree(dnsmi::pnet_forward(din, H, dout, B, static_cast<const uint16_t*>(X), params,
-                                     static_cast<uint16_t*>(wb), wf, static_cast<uint16_t*>(wh), Y,
+                                     static_cast<uint16_t*>(wb), static_cast<uint16_t*>(wh), Y,
                                      as_stream(stream)),
                  "pnet_forward");
 }
@@ -464,16 +463,16 @@ int dnsmi_pnet_features(dnsmi_ctx* ctx, const double* n_m2, const double* n_m1, 
 
 int dnsmi_guess_profile(dnsmi_ctx* ctx, const double* state, double* pred, double* rhs_prev,
                         const float* hist1, float* hist2, int din, int H, int dout, const float* params,
-                        void* wb, void* X, float* wf, void* wh, float* Y, float s_1, float s_2, float s_out,
+                        void* wb, void* X, float* /*wf*/, void* wh, float* Y, float s_1, float s_2, float s_out,
                         void* stream) {
   DNSMI_CHECK_CTX(ctx)
-  DNSMI_REQUIRE(state && pred && rhs_prev && hist1 && hist2 && params && wb && X && wf && wh && Y,
+  DNSMI_REQUIRE(state && pred && rhs_prev && hist1 && hist2 && params && wb && X && wh && Y,
                 "guess_profile: null pointer");
   DNSMI_REQUIRE(dnsmi_pnet_params(din, H, dout) > 0, "guess_profile: din a multiple of 32, H of 64");
   DNSMI_REQUIRE((const void*)state != pred && (void*)pred != rhs_prev && (const void*)hist1 != hist2,
                 "guess_profile: buffers must be distinct");
   return dnsmi::guess_walls_profile(c, state, pred, rhs_prev, hist1, hist2, din, H, dout, params,
-                                    static_cast<uint16_t*>(wb), static_cast<uint16_t*>(X), wf,
+                                    static_cast<uint16_t*>(wb), static_cast<uint16_t*>(X),
                                     static_cast<uint16_t*>(wh), Y, s_1, s_2, s_out, as_stream(stream));
 }
 

@@ -598,9 +598,8 @@ static int pn_cast(const PNet& net, const float* prm, uint16_t* wb, hipStream_t 
   return hipGetLastError() == hipSuccess ? DNSMI_OK : DNSMI_EHIP;
 }
 
-int pnet_forward(int din, int H, int dout, int B, const uint16_t* X, const float* prm, uint16_t* wb,
-                 float* /*wf: the pre-activations, which only training keeps*/, uint16_t* wh, float* Y,
-                 hipStream_t s) {
+int pnet_forward(int din, int H, int dout, int B, const uint16_t* X, const float* prm, uint16_t* wb, uint16_t* wh,
+                 float* Y, hipStream_t s) {
   const PNet net{din, H, dout};
   if (!pn_ok(net) || B <= 0) return DNSMI_EINVAL;
   uint16_t* H1 = wh;
@@ -690,8 +689,7 @@ static GemmArgs pn_dz(int B, int N, int K, const uint16_t* dQ, const uint16_t* W
 // column sum (one thread per column) or loss sum (one thread) per launch and
 // the batch never split.
 int pnet_grad(int din, int H, int dout, int B, const uint16_t* X, const float* T, const float* prm,
-              uint16_t* wb, float* wf, uint16_t* wh, float* /*part: the loss's parts live in wf*/, float* grad,
-              float* loss, hipStream_t s) {
+              uint16_t* wb, float* wf, uint16_t* wh, float* grad, float* loss, hipStream_t s) {
   const PNet net{din, H, dout};
   if (!pn_ok(net) || B <= 0) return DNSMI_EINVAL;
   float* Z1 = wf;
@@ -911,11 +909,11 @@ int extrap_walls(Ctx* c, const double* n0, const float* h1, float* h2, double* n
 // its output, then N_ext = quadratic extrapolation + s_out Y / w into
 // rhs_prev (h2 <- N^n) and pred = the predictor's solve fed with N_ext.
 // Caller-owned buffers, M = the number of modes: wb (the bf16 weight
-// copies, one word per parameter), X (M din bf16 words), wf (2 H M floats),
-// wh (2 H M bf16 words), Y (M dout floats).
+// copies, one word per parameter), X (M din bf16 words), wh (2 H M bf16 words),
+// Y (M dout floats).
 int guess_walls_profile(Ctx* c, const double* state, double* pred, double* rhs_prev, const float* h1, float* h2,
-                        int din, int H, int dout, const float* prm, uint16_t* wb, uint16_t* X, float* wf,
-                        uint16_t* wh, float* Y, float s_1, float s_2, float s_out, hipStream_t s) {
+                        int din, int H, int dout, const float* prm, uint16_t* wb, uint16_t* X, uint16_t* wh,
+                        float* Y, float s_1, float s_2, float s_out, hipStream_t s) {
   if (!c->walls) return c->fail(DNSMI_EINVAL, "profile network: plane Couette contexts only");
   if (dout != 6 * c->ny) return c->fail(DNSMI_EINVAL, "profile network: dout must be 6 ny");
   const long long M = (long long)c->Nz1 * c->Nx1;
@@ -928,7 +926,7 @@ int guess_walls_profile(Ctx* c, const double* state, double* pred, double* rhs_p
   hipLaunchKernelGGL(k_pn_features_hist, dim3(nb), dim3(256), 0, s, a, reinterpret_cast<const cx<double>*>(c->rhs0),
                      reinterpret_cast<const float2*>(h1), reinterpret_cast<const float2*>(h2), X);
   if ((rc = check_launch(c, "profile input"))) return rc;
-  if ((rc = pnet_forward(din, H, dout, (int)M, X, prm, wb, wf, wh, Y, s)))
+  if ((rc = pnet_forward(din, H, dout, (int)M, X, prm, wb, wh, Y, s)))
     return c->fail(rc, "profile network forward");
   if ((rc = extrap_walls(c, c->rhs0, h1, h2, rhs_prev, nullptr, nullptr, 32, s_1, s_2, s_out, 3, s))) return rc;
   hipLaunchKernelGGL(k_pn_apply, dim3(nb), dim3(256), 0, s, a, Y, reinterpret_cast<cx<double>*>(rhs_prev));

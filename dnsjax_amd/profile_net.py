@@ -90,9 +90,8 @@ class ProfileNet:
         B = X.shape[0]
         wf = self._buf("wf", B * (2 * self.H + self.dout), torch.float32)
         wh = self._buf("wh", B * (3 * self.H + self.dout), torch.int16)
-        part = self._buf("part", (B * self.dout + 255) // 256, torch.float32)
         _lib.check(self.lib.dnsmi_pnet_grad(self.din, self.H, self.dout, B, _ptr(X), _ptr(T), _ptr(self.params),
-                                            _ptr(self.wb), _ptr(wf), _ptr(wh), _ptr(part), _ptr(self.grad),
+                                            _ptr(self.wb), _ptr(wf), _ptr(wh), None, _ptr(self.grad),
                                             _ptr(self.loss), _stream()))
         return self.loss
 
@@ -103,24 +102,22 @@ class ProfileNet:
 
     def forward(self, X: torch.Tensor) -> torch.Tensor:
         B = X.shape[0]
-        wf = self._buf("wf", B * 2 * self.H, torch.float32)
         wh = self._buf("wh", B * 2 * self.H, torch.int16)
         Y = torch.empty((B, self.dout), dtype=torch.float32, device=self.device)
         _lib.check(self.lib.dnsmi_pnet_forward(self.din, self.H, self.dout, B, _ptr(X), _ptr(self.params),
-                                               _ptr(self.wb), _ptr(wf), _ptr(wh), _ptr(Y), _stream()))
+                                               _ptr(self.wb), None, _ptr(wh), _ptr(Y), _stream()))
         return Y
 
     def guess(self, nat, state, pred, rhs_prev, hist1, hist2, scales: Scales) -> None:
         """The plane Couette guess of ``dnsmi_guess_profile`` (hist2 <- N^n)."""
         M = nat.shape[1] * nat.shape[2]
         X = self._buf("gX", M * self.din, torch.int16)
-        wf = self._buf("gwf", M * 2 * self.H, torch.float32)
         wh = self._buf("gwh", M * 2 * self.H, torch.int16)
         Y = self._buf("gY", M * self.dout, torch.float32)
         s_1, s_2, s_out = scales.astuple()
         nat._chk(self.lib.dnsmi_guess_profile(nat.handle, _ptr(state), _ptr(pred), _ptr(rhs_prev), _ptr(hist1),
                                               _ptr(hist2), self.din, self.H, self.dout, _ptr(self.params),
-                                              _ptr(self.wb), _ptr(X), _ptr(wf), _ptr(wh), _ptr(Y), s_1, s_2,
+                                              _ptr(self.wb), _ptr(X), None, _ptr(wh), _ptr(Y), s_1, s_2,
                                               s_out, _stream()))
 
 

@@ -336,11 +336,11 @@ int dnsmi_step_device_guess(dnsmi_ctx* ctx, const double* state, double* next, d
 long long dnsmi_pnet_params(int din, int H, int dout); /* -1 if unsupported */
 /* Gradient of L = (1/(B dout)) sum (Y - T)^2 over X (B,din) bf16, T (B,dout)
  * FP32 into grad (FP32), loss into loss_dev (may be NULL).  Work: wf
- * B (2H + dout) floats, wh B (3H + dout) words, part ceil(B dout/256)
- * floats (not used: the partial sums live in wf). */
+ * B (2H + dout) floats, wh B (3H + dout) words; part is not used (may be
+ * NULL). */
 int dnsmi_pnet_grad(int din, int H, int dout, int B, const void* X, const float* T, const float* params,
                     void* wb, float* wf, void* wh, float* part, float* grad, float* loss_dev, void* stream);
-/* Y (B,dout) = net(X); work wf 2 H B floats, wh 2 H B words. */
+/* Y (B,dout) = net(X); work wh 2 H B words; wf is not used (may be NULL). */
 int dnsmi_pnet_forward(int din, int H, int dout, int B, const void* X, const float* params, void* wb,
                        float* wf, void* wh, float* Y, void* stream);
 /* One Adam step over P parameters (beta1 0.9, beta2 0.999, eps 1e-8). */
@@ -358,8 +358,8 @@ int dnsmi_pnet_features(dnsmi_ctx* ctx, const double* n_m2, const double* n_m1, 
  * the step's reference) into the context, rhs_prev = quadratic
  * extrapolation plus s_out Y / w per point, pred = the predictor's solve fed
  * with rhs_prev, hist2 <- N^n.  Work, M = (nz-1) nx/2 modes: X M din words,
- * wf 2 H M floats, wh 2 H M words, Y M dout floats, wb one word per
- * parameter. */
+ * wh 2 H M words, Y M dout floats, wb one word per parameter; wf is not used
+ * (may be NULL). */
 int dnsmi_guess_profile(dnsmi_ctx* ctx, const double* state, double* pred, double* rhs_prev,
                         const float* hist1, float* hist2, int din, int H, int dout, const float* params,
                         void* wb, void* X, float* wf, void* wh, float* Y, float s_1, float s_2, float s_out,
