@@ -36,7 +36,6 @@ __device__ __forceinline__ uint16_t pn_bf16(float f) {
   const uint32_t u = __float_as_uint(f);
   return (uint16_t)((u + (((u >> 16) & 1u) + 0x7FFFu)) >> 16);
 }
-__device__ __forceinline__ float pn_float(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 __device__ __forceinline__ float pn_silu(float z) { return z / (1.0f + __expf(-z)); }
 __device__ __forceinline__ float pn_dsilu(float z) {
   const float s = 1.0f / (1.0f + __expf(-z));
@@ -515,10 +514,6 @@ struct PNet {
   __host__ __device__ long long w3() const { return b2() + H; }
   __host__ __device__ long long b3() const { return w3() + (long long)H * dout; }
   __host__ __device__ long long n() const { return b3() + dout; }
-  // work floats for a batch of B: Z1, Z2 (B H each), Y / dY (B dout)
-  __host__ __device__ long long work_f(int B) const { return (long long)B * (2 * H + dout); }
-  // work bf16 words: H1, H2, dZ (B H each), dY (B dout)
-  __host__ __device__ long long work_h(int B) const { return (long long)B * (3 * H + dout); }
 };
 
 // bf16 copies of the parameters, four per thread.
