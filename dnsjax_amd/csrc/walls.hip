@@ -1244,7 +1244,7 @@ struct ImmArgs {
   const cx<double>* uj;   // velocity_j
   const cx<double>* nn;   // nonlin_n
   const cx<double>* nj;   // nonlin_j
-  cx<double>* out;        // velocity_new (may alias uj)
+  cx<double>* out;        // velocity_new (may alias un or uj)
   cx<double>* corr;       // correction (may be null)
   double* partials;       // per-block sum of quadrature-weighted k_metric |delta|^2
   const double *d1w, *d2w, *qw;  // stencil weights as [k][y]
@@ -2252,6 +2252,12 @@ static int launch_imm(Ctx* c, const ImmArgs& a, hipStream_t s) {
   return DNSMI_OK;
 }
 
+// `out` may alias un or uj: a mode's new velocity is stored by the workgroup
+// that read the mode's rows (phase 5 reads a point of uj and then stores it),
+// after the last of its reads of u^n.  In the one-launch form all of those,
+// the absent second mode's repeats of the first one's rows among them, come
+// before the barriers in front of phase 5; the five-launch form's are in
+// earlier launches.
 static int walls_imm(Ctx* c, const double* un, const double* uj, const double* nn,
                      const double* nj, double* out, double* corr, double* err, hipStream_t s) {
   WallTables* t = c->wt;
@@ -2314,8 +2320,9 @@ static int walls_autotune(Ctx* c) {
   if (hipMemset(c->rhs0, 0, c->spec_elems * 16) != hipSuccess ||
       hipMemset(c->bufA, 0, c->spec_elems * 16) != hipSuccess)
     return c->fail(DNSMI_EHIP, "autotune: memset");
-  // zero fields in, the new velocity into a buffer of its own (the fused
-  // form needs it apart from u^n); bufA is transform scratch, unused here
+  // zero fields in, the new velocity into a buffer of its own (in place, the
+  // second call would no longer start from zeros); bufA is transform scratch,
+  // unused here
   double* z = c->rhs0;
   double* o = static_cast<double*>(c->bufA);
   hipEvent_t e0, e1;
