@@ -254,6 +254,10 @@ __host__ __device__ constexpr int high_operands(int p, bool back, bool mx) {
 __host__ __device__ constexpr int low_operands(int p, bool back, bool mx) {
   return back || !mx ? 4 : chunk_span(p, back, mx) / 4;
 }
+// Longest column of the chunked solves: the five-launch form's H_k solve keeps
+// six of them with their zero rows (chunk_lds) in LDS, at most 65392 bytes for
+// every Ny up to here.
+constexpr int kChunkNy = 650;
 __host__ __device__ constexpr int map_operands(int p, bool back, bool mx) {
   return (high_operands(p, back, mx) + low_operands(p, back, mx) + 1) / 2 * 2;
 }
@@ -827,10 +831,7 @@ int walls_setup(Ctx* c) {
   const bool mx = c->fp32_primary;
   const size_t nf = (size_t)chunk_count(Ny, p, false, mx) * U * map_words(p, false, mx),
                nb = (size_t)chunk_count(Ny, p, true, mx) * U * map_words(p, true, mx);
-  // the chunked solve also stages three right-hand sides per mode pair in
-  // LDS (2 * 3 * (Ny + 32) complex values), which must fit in 64 KiB
-  const bool maps_fit = nf < (1ull << 28) && nb < (1ull << 28) &&
-                        (size_t)2 * 3 * (Ny + 32) * sizeof(cx<double>) <= 65536;
+  const bool maps_fit = nf < (1ull << 28) && nb < (1ull << 28) && Ny <= kChunkNy;
   const bool forced = g.tile_cols != 0;  // the variant bits choose the form
   if (forced && (g.variants & 8) == 0 && !maps_fit)
     return c->fail(DNSMI_EINVAL,
@@ -1612,8 +1613,9 @@ __global__ void __launch_bounds__(kSweepLanes)
 // overwrite rows that have left the window), and results go back there, off
 // the chain.
 //
-// Bound: the products, 27 ns each and one per SIMD at a time, 128 + 156 of
-// them for a solve at Ny = 256, p = 6 (7.6 us), where broadcasting the window to
+// Bound, with the maps in a cache near by: the products, 27 ns each and one per
+// SIMD at a time, 128 + 156 of them for a solve at Ny = 256, p = 6 (7.6 us; in
+// the whole step the maps' way there sets the pace, k_imm_fused), where broadcasting the window to
 // one lane per map row through LDS took 50 FMA steps behind 150 LDS reads per
 // 16 rows (1.5 us).  Windows of 16 rows (12 to 8 new ones each) take fewer
 // products per row than two-tile ones of 16 new rows (p = 4: 0.83 against
@@ -1851,8 +1853,8 @@ __global__ void __launch_bounds__(64, 2)
 //
 // Traffic: 15 vector components, and a class's maps for every two modes (1140
 // bytes per point at p = 6, where the fields of both are 480).  The maps' way from the
-// caches is the bound, not the products, which would take 20 us per item at
-// Ny = 256, p = 6; four items per CU (36 KB of LDS, 256 registers) put one
+// caches is the bound, not the products, which would take 15 us per item (two
+// solves) at Ny = 256, p = 6; four items per CU (36 KB of LDS, 256 registers) put one
 // solving wavefront on each SIMD (the first wavefronts of a CU's workgroups
 // start on different ones).  One predictor, with the sequence of launches that
 // was the fastest before: 128 x 256 x 128, p = 6, five launches 623 us, so
@@ -1860,7 +1862,10 @@ __global__ void __launch_bounds__(64, 2)
 // each wavefront) 68 us, so 27 us; 48 x 65 x 32, p = 4: 35 us, so 12 us.
 // Mixed contexts (MX; chunk_tiles): 128 x 256 x 128, p = 6, 563 us, so 336 us.
 constexpr int kImmRows = 4;       // LDS rows per mode
-constexpr int kImmFusedNy = 278;  // largest Ny of the fused form
+// Largest Ny of the one-launch form.  LDS (8 rows, 40 KB) and points per lane
+// would reach 320; five points a lane (from 257) already spill up to 53
+// registers, and longer columns have neither been measured nor taken.
+constexpr int kImmFusedNy = 278;
 
 template <int PO, int YP, bool MX>
 __global__ void __launch_bounds__(128, 2)
@@ -2294,8 +2299,7 @@ static int walls_imm(Ctx* c, const double* un, const double* uj, const double* n
   {
     if (!c->sweep_seq && !t->lk_fmap) return c->fail(DNSMI_EINVAL, "imm: chunk maps not built");
     ProfScope ps(c, KID_W_IMM, s);
-    if (4 * (size_t)t->Ny * sizeof(cx<double>) > 65536 ||
-        (!c->sweep_seq && (size_t)2 * 3 * (t->Ny + 32) * sizeof(cx<double>) > 65536))
+    if (4 * (size_t)t->Ny * sizeof(cx<double>) > 65536 || (!c->sweep_seq && t->Ny > kChunkNy))
       return c->fail(DNSMI_EINVAL, "imm: ny too large for the per-mode LDS rows");
     int rc = DNSMI_OK;
     switch (t->p) {
