@@ -468,7 +468,7 @@ static int pn_tiles(int M, int N, int BM, int BN) { return (int)(((long long)M +
 // 64 (four).  8128 x 3104 -> 256, 254 workgroups of 64 x 128: 36 us, 64 x 64
 // tiles 40 us, 64 x 128 in four waves 39 us; 2048 x 3104 -> 256: 18 us in 256
 // workgroups of 32 x 64, where 64 x 128 would fill 64 CUs.
-static bool pn_large(int M, int N) { return N > 64 && pn_tiles(M, N, 64, 128) >= 208; }
+static bool pn_large(int M, int N) { return N >= 128 && pn_tiles(M, N, 64, 128) >= 208; }
 static int pn_layer_tiles(int M, int N) { return pn_large(M, N) ? pn_tiles(M, N, 64, 128) : pn_tiles(M, N, 32, 64); }
 
 // Chunks in flight (S): four where K is long (the input layer: 36 -> 34 us at
@@ -495,7 +495,7 @@ static int pn_layer(const GemmArgs& g, hipStream_t s) {
 static int pn_back(const BackArgs& a, hipStream_t s) {
   const int n = a.nz + a.nw + a.ns + (a.loss.out ? 1 : 0);
   if (!n) return DNSMI_OK;
-  if (a.w.N > 64)
+  if (a.w.N >= 128)
     hipLaunchKernelGGL(k_pn_back<128>, dim3(n), dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL(k_pn_back<64>, dim3(n), dim3(256), 0, s, a);
@@ -625,7 +625,10 @@ struct WGrad {
 static WGrad pn_wgrad(int M, int N, int B, const uint16_t* P, const uint16_t* Q, float* G, float* scratch,
                       long long room, int want) {
   WGrad r{};
-  const int tiles = pn_tiles(M, N, 64, N > 64 ? 128 : 64);
+  // 128 columns a tile only where the matrix has them: a narrower one is loaded
+  // element by element throughout (pn_tile).  Gradient of 8128 samples, 256 ->
+  // 126 outputs: 121 us in tiles of 128, 103 us of 64.
+  const int tiles = pn_tiles(M, N, 64, N >= 128 ? 128 : 64);
   const long long n = (long long)(M + 1) * N;
   long long parts = want / tiles;
   if (parts > (B + 127) / 128) parts = (B + 127) / 128;
