@@ -223,9 +223,9 @@ static void band_solve(const Band& B, std::vector<double>& b) {
 // one order of operations to the bit: chunks of 16 rows, each of a map's sums
 // over the window's rows in ascending order (v_mfma_f64_16x16x4_f64 is four
 // fused multiply-adds in ascending k), and the right-hand sides' terms one by
-// one (imm_fhat_mx_at, imm_r_at).  Its maps take 80 words per row of the
-// column where the FP64 contexts' take 53 (p = 4; p = 6: 96 and 70), and one step
-// of 128 x 256 x 128, p = 6, 336 us where theirs takes 296.
+// one (imm_fhat_mx_at, imm_r_at).  Its maps take 72 words per row of the
+// column where the FP64 contexts' take 53 (p = 4; p = 6: 80 and 70), and one step
+// of 128 x 256 x 128, p = 6, 317 us where theirs takes 302.
 __host__ __device__ constexpr int chunk_tiles(int p, bool back, bool mx) { return mx || (back && p >= 6) ? 2 : 1; }
 __host__ __device__ constexpr int chunk_keep(int p, bool back) { return back ? 2 * p : p; }
 __host__ __device__ constexpr int chunk_rows(int p, bool back, bool mx) {
@@ -247,9 +247,13 @@ __host__ __device__ constexpr int chunk_count(int n, int p, bool back, bool mx) 
 // is 1 KB of consecutive words.  One tile: e = k / 4, entry (t = r, k = 4 e +
 // g).  Two: first the operands of rows 16 + r (high_operands), then those of
 // rows r (low_operands), of which a back map's k >= 16 are zero by construction
-// (it is lower triangular) and left out; an odd count is filled up with zeros.
+// (it is lower triangular) and left out.  A mixed context's back map is the
+// identity in rows and columns >= 16 (its steps eliminate with rows < 16 only):
+// those columns are left out too, and the window's rows added at their place in
+// the sum (chunk_chain), the same value to the bit: one step of 128 x 256 x 128,
+// p = 6, 360 us with them, 317 us without.
 __host__ __device__ constexpr int high_operands(int p, bool back, bool mx) {
-  return chunk_tiles(p, back, mx) == 1 ? 0 : chunk_span(p, back, mx) / 4;
+  return chunk_tiles(p, back, mx) == 1 ? 0 : back && mx ? 4 : chunk_span(p, back, mx) / 4;
 }
 __host__ __device__ constexpr int low_operands(int p, bool back, bool mx) {
   return back || !mx ? 4 : chunk_span(p, back, mx) / 4;
@@ -259,11 +263,11 @@ __host__ __device__ constexpr int low_operands(int p, bool back, bool mx) {
 // every Ny up to here.
 constexpr int kChunkNy = 650;
 __host__ __device__ constexpr int map_operands(int p, bool back, bool mx) {
-  return (high_operands(p, back, mx) + low_operands(p, back, mx) + 1) / 2 * 2;
+  return high_operands(p, back, mx) + low_operands(p, back, mx);
 }
 __host__ __device__ constexpr int map_words(int p, bool back, bool mx) { return 64 * map_operands(p, back, mx); }
 __host__ __device__ constexpr int map_word(int e, int lane) { return ((e >> 1) * 64 + lane) * 2 + (e & 1); }
-// entry (t, k) of word i (k past the window where it is filled up)
+// entry (t, k) of word i
 __host__ __device__ inline void map_entry(int i, int high, int& t, int& k) {
   const int e = (i >> 7) * 2 + (i & 1), lane = (i & 127) >> 1;
   t = (lane & 15) + (e < high ? 16 : 0);
@@ -277,8 +281,8 @@ __host__ __device__ inline void map_entry(int i, int high, int& t, int& k) {
 // cB, applies the steps j = T, T - 1, ... (at most B, j >= 0: divide by the
 // diagonal, eliminate upwards) to the window of rows T - t, t < W = B + kl +
 // ku.  Written as map u of U; `raw(r, j)` reads the factored band, `piv(j)`
-// the pivot row.  Returns false if an entry left out is not zero (it cannot
-// be, by the argument above; the check keeps the layout honest).
+// the pivot row.  Returns false if an entry left out is not what it is taken for
+// (it cannot be, by the argument above; the check keeps the layout honest).
 template <typename Raw, typename Piv>
 static bool chunk_maps(int n, int p, bool mx, int u, int U, Raw raw, Piv piv, double* F, double* G) {
   const int kl = p, kuu = 2 * p;
@@ -286,15 +290,16 @@ static bool chunk_maps(int n, int p, bool mx, int u, int U, Raw raw, Piv piv, do
   std::vector<double> X;
   auto write = [&](bool back, int c, double* out) {
     const int W = chunk_window(p, back, mx), words = map_words(p, back, mx), high = high_operands(p, back, mx);
-    const int klow = 4 * low_operands(p, back, mx);  // columns that rows 0 .. 15 keep
+    const int klow = 4 * low_operands(p, back, mx);  // columns that rows 0 .. 15 keep, and the others
+    const int khigh = 4 * high;
     double* m = out + ((size_t)c * U + u) * words;
     for (int i = 0; i < words; ++i) {
       int t, k;
       map_entry(i, high, t, k);
       m[i] = t < W && k < W ? X[(size_t)t * W + k] : 0.0;
     }
-    for (int t = 0; t < 16 && t < W; ++t)
-      for (int k = klow; k < W; ++k) ok = ok && X[(size_t)t * W + k] == 0.0;
+    for (int t = 0; t < W; ++t)
+      for (int k = t < 16 ? klow : khigh; k < W; ++k) ok = ok && X[(size_t)t * W + k] == (t == k ? 1.0 : 0.0);
   };
   for (int c = 0; c < chunk_count(n, p, false, mx); ++c) {
     const int B = chunk_rows(p, false, mx), W = chunk_window(p, false, mx), j0 = c * B;
@@ -656,7 +661,7 @@ __global__ void __launch_bounds__(64) k_setup_maps(GpuSetup g, double* lf, doubl
     }
   }
   const int words = map_words(kl, back, mx), high = high_operands(kl, back, mx);
-  const int klow = 4 * low_operands(kl, back, mx);
+  const int klow = 4 * low_operands(kl, back, mx), khigh = 4 * high;
   double* F = (which == 0 ? (back ? lb : lf) : (back ? hb : hf)) + ((size_t)c * g.U + u) * words;
   for (int i = lane; i < words; i += 64) {
     int t, k;
@@ -664,8 +669,10 @@ __global__ void __launch_bounds__(64) k_setup_maps(GpuSetup g, double* lf, doubl
     F[i] = t < W && k < W ? X[t * W + k] : 0.0;
   }
   bool bad = false;
-  for (int e = lane; e < 16 * (W - klow); e += 64)
-    bad = bad || ((e & 15) < W && X[(e & 15) * W + klow + (e >> 4)] != 0.0);
+  for (int e = lane; e < W * W; e += 64) {
+    const int t = e / W, k = e % W;
+    bad = bad || (k >= (t < 16 ? klow : khigh) && X[e] != (t == k ? 1.0 : 0.0));
+  }
   if (bad) g.flag[1] = 1;
 }
 
@@ -1666,7 +1673,7 @@ struct MapChunk {
 };
 
 // Chunks of maps in registers, loaded that many less one ahead: eight words a
-// lane each in one-tile windows, 20 to 24 in two-tile ones.
+// lane each in one-tile windows, 16 to 24 in two-tile ones.
 template <int PO, bool BACK, bool MX>
 struct ChunkMaps {
   static constexpr int R = chunk_tiles(PO, BACK, MX) == 1 ? 4 : 3, N = map_operands(PO, BACK, MX);
@@ -1741,6 +1748,10 @@ __device__ __forceinline__ void chunk_chain(const double* __restrict__ map, int 
       if (KR + e < WR) fresh[KR + e < WR ? KR + e : 0] = in[2 * S * 4 * (KR + e)];
       if (e == 0 && KEEP % 4 != 0) fresh[KR - 1] = in[2 * S * 4 * (KR - 1)];
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (MX && BACK) {  // rows and columns >= 16: the identity
+#pragma unroll
+      for (int i = 0; i < KR; ++i) acc[1][i] += w[BR + i];
     }
 #pragma unroll
     for (int i = 0; i < BR; ++i) done[i] = acc[i >> 2][i & 3];
@@ -1860,7 +1871,7 @@ __global__ void __launch_bounds__(64, 2)
 // was the fastest before: 128 x 256 x 128, p = 6, five launches 623 us, so
 // 296 us; 64 x 128 x 64, p = 4, two launches (solve and parallel phases by
 // each wavefront) 68 us, so 27 us; 48 x 65 x 32, p = 4: 35 us, so 12 us.
-// Mixed contexts (MX; chunk_tiles): 128 x 256 x 128, p = 6, 563 us, so 336 us.
+// Mixed contexts (MX; chunk_tiles): 128 x 256 x 128, p = 6, 563 us, so 317 us.
 constexpr int kImmRows = 4;       // LDS rows per mode
 // Largest Ny of the one-launch form.  LDS (8 rows, 40 KB) and points per lane
 // would reach 320; five points a lane (from 257) already spill up to 53
