@@ -142,7 +142,8 @@ def measured_traffic(kernel: str, b: int, mode: str = "2"):
     t = "double" if b == 16 else "float"
     args = {"y_inverse": f"{t}, 192, 16, true, 0", "x_nonlinear": f"{t}, 192, 16, 0",
             "y_forward": f"{t}, 192, 16, {mode}, true"}.get(kernel, f"{t}, 192, 16")
-    ent = json.load(open(path))["kernels"].get(f"k_{kernel}<{args}>")
+    name = "y_forward_serial" if kernel == "y_forward" else kernel  # the form it takes at 128^3
+    ent = json.load(open(path))["kernels"].get(f"k_{name}<{args}>")
     return int(ent["traffic_bytes"]) if ent else None
 
 
